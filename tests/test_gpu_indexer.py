@@ -203,6 +203,43 @@ def test_dsa_paged_mqa_logits():
             assert np.array_equal(got[~fin & ~np.isinf(want)], want[~fin & ~np.isinf(want)])
 
 
+@pytest.mark.parametrize('heads,dim,block,msl', [
+    (32, 128, 64, 640), (64, 128, 32, 2083), (64, 64, 128, 1), (128, 64, 96, 31), (32, 256, 64, 33), (96, 64, 256, 4096),
+    (32, 128, 48, 500), (64, 256, 64, 300), (128, 128, 64, 300)])
+def test_dsa_paged_logits_edges(heads, dim, block, msl):
+    """Lengths at the edges of 32-key blocks, pages and the table, negative and out-of-range table entries (the first
+    reads page 0, the others no key), page sizes off the 32-key grid and head counts past the register budget; every
+    logit within the FP32 summation bound."""
+    g = torch.Generator().manual_seed(heads + dim + block + msl)
+    lens = torch.tensor([0, 1, 31, 32, 33, block - 1, block, block + 1, msl - 1, msl, msl + 500], dtype=torch.int32)
+    rows, width, pages = len(lens), max(1, -(-msl // block)), 37
+    vals = _fp8((pages, block, dim), g)
+    scl = torch.rand(pages, block, generator=g) + 0.5
+    kv = torch.empty(pages, block * (dim + 4), dtype=torch.uint8)
+    kv[:, :block * dim] = vals.view(torch.uint8).reshape(pages, -1)
+    kv[:, block * dim:] = scl.view(torch.uint8).reshape(pages, -1)
+    table = torch.randint(0, pages, (rows, width), generator=g, dtype=torch.int32)
+    table[2, 0], table[9, width // 2], table[10, width - 1] = -1, pages, 2 ** 31 - 1
+    q, w = _fp8((rows, 1, heads, dim), g), torch.randn(rows, heads, generator=g)
+    for clean in (False, True):
+        got = ops.dsa_paged_mqa_logits(q.cuda(), kv.view(pages, block, 1, dim + 4).cuda(), w.cuda(), lens.cuda(),
+                                       table.cuda(), None, msl, clean).cpu().numpy().astype(np.float64)
+        fill = -np.inf if clean else 0.0
+        for r in range(rows):
+            n = min(int(lens[r]), msl, width * block)
+            page = table[r].clamp(min=0).long().repeat_interleave(block)[:n]
+            live = (page < pages).numpy()
+            page = page.clamp(max=pages - 1)
+            at = torch.arange(n) % block
+            k, ks = vals[page, at].float().numpy().astype(np.float64), scl[page, at].numpy().astype(np.float64)
+            qd, wd = q[r, 0].float().numpy().astype(np.float64), w[r].numpy().astype(np.float64)
+            want = np.where(live, (np.maximum(qd @ k.T, 0) * wd[:, None]).sum(0) * ks, fill)
+            bound = (dim + heads + 4) * 2.0 ** -24 * ((np.abs(qd) @ np.abs(k).T) * np.abs(wd)[:, None]).sum(0) * ks
+            same = got[r, :n] == want
+            assert (same | (np.abs(got[r, :n] - np.where(np.isinf(want), 0, want)) <= bound + 1e-30)).all(), r
+            assert (got[r, n:] == fill).all(), r
+
+
 def test_glm_schedule_and_sm_count():
     assert glm.get_paged_mqa_logits_metadata(None, 1, 2, x=3) is None
     assert glm.get_num_sms(None) == torch.cuda.get_device_properties(0).multi_processor_count

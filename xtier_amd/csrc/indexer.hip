@@ -645,7 +645,8 @@ struct DsaArgs {
 
 constexpr int kDsaWaves = 4;
 
-// Workgroup = (4 query rows, one per wavefront, keys_per_wg keys); the wavefronts walk the same 32-key blocks, so a
+// The shapes the two kernels below do not take (query and weights past their registers, pages off the 32-key grid, rows
+// off 16-byte alignment). Workgroup = (4 query rows, one per wavefront, keys_per_wg keys); the wavefronts walk the same 32-key blocks, so a
 // block's key bytes are fetched once for the four rows. Per block and 32-head group, S = Q . K^T on 32x32x16 FP16
 // MFMAs of the converted E4M3 values (A = Q: lane (head l % 32, dims 16kk + 8 (l / 32) .. +7); B = K^T: lane (key
 // l % 32, same dims); C: lane (key column l % 32, heads 8 (r / 4) + 4 (l / 32) + r % 4)).
@@ -800,6 +801,105 @@ __global__ __launch_bounds__(64 * kDsaWaves) void dsa_flat_kernel(const DsaArgs 
   }
 }
 
+// Paged keys whose pages hold a multiple of 32 keys (decode): one row per workgroup, `bpw` consecutive 32-key blocks
+// per wavefront, so a batch of a few rows still spreads over every CU. The row's query (as FP16) and head weights stay
+// in registers for the wavefront's whole range; a block's page is uniform, so the wavefront's table entries are one
+// vector load before the loop and a block's address is scalar. Bound: HBM, D + 4 bytes per key; a wavefront keeps one
+// block's loads in flight beyond the one it computes (two or three measured 21.3 us against 20.8). k-step kk covers dims h D/2 + 8 kk .. + 7 in both operands (not
+// 16 kk + 8 h), so a lane reads its half of a key's row as 16-byte pieces. Measured at 32 rows x 32 heads x 128, up to
+// 32768 keys each (16.6K in the mean, 69 MB): 20.8 us = 3.3 TB/s against 352 us for dsa_logits_kernel, which puts four rows in a workgroup
+// and 4096 keys in a wavefront's serial walk.
+constexpr int kDsaAhead = 1;
+
+template <int NK, int G>
+__global__ __launch_bounds__(64 * kDsaWaves) void dsa_paged_kernel(const DsaArgs a, int bpw) {
+  constexpr int D = 16 * NK, PIECES = D / 32;   // 16-byte pieces of a lane's half row
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+  const int row = blockIdx.y;
+  const int b0 = __builtin_amdgcn_readfirstlane(((int)blockIdx.x * kDsaWaves + wave) * bpw);   // first 32-key block
+  const int cols = a.out_cols, n_blocks = min(bpw, (cols + 31) / 32 - b0);
+  if (n_blocks <= 0) return;   // no barrier below
+  const int len = uniform_load(a.ke + row), width = a.bt_width * (a.block / 32);
+  const int lim = min(len, width <= 0x3FFFFFF ? width * 32 : 0x7FFFFFFF);
+  const int live_blocks = min(n_blocks, (max(lim, 0) + 31) / 32 - b0);
+  const float fill = a.clean ? -__builtin_inff() : 0.0f;
+  float* out = a.logits + (int64_t)row * a.ld;
+  // table entries of this range: lane i holds that of block b0 + i; a negative one reads page 0, as the reference's
+  // clamp does (indexer_torch.py:61), and one past the cache reads as no key
+  const int bpp = a.block / 32;   // 32-key blocks per page
+  int page = 0;
+  if (lane < live_blocks) page = max(a.block_table[(int64_t)row * a.bt_stride + (b0 + lane) / bpp], 0);
+  half8_t qf[G][NK];
+  float wv[G][16];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const uint8_t* qp = a.q + (int64_t)row * a.q_rs + (int64_t)(32 * g + j) * a.q_hs + h * (D / 2);
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) qf[g][kk] = fp8x8_to_f16(*reinterpret_cast<const uint64_t*>(qp + 8 * kk));
+    const float* wp = a.w + (int64_t)row * a.w_rs + 32 * g + 4 * h;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) wv[g][r] = wp[8 * (r >> 2) + (r & 3)];
+  }
+  uint4 raw[kDsaAhead + 1][PIECES];
+  float ksc[kDsaAhead + 1];
+  auto load = [&](int i, int slot) {   // block i of the range
+    const int pg_i = __builtin_amdgcn_readlane(page, i);
+    const int in = (b0 + i) % bpp * 32;   // first key within the page
+    const uint8_t* pg = a.k + (int64_t)(pg_i < a.num_pages ? pg_i : 0) * a.page_bytes;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p)
+      raw[slot][p] = *reinterpret_cast<const uint4*>(pg + (uint32_t)((in + j) * D + h * (D / 2) + 16 * p));
+    ksc[slot] = *reinterpret_cast<const float*>(pg + (uint32_t)(a.block * D + 4 * (in + j)));
+  };
+  auto compute = [&](int i, int slot) {
+    float acc = 0.0f;
+    half8_t kv[NK];
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      kv[2 * p] = fp8x8_to_f16((uint64_t)raw[slot][p].x | ((uint64_t)raw[slot][p].y << 32));
+      kv[2 * p + 1] = fp8x8_to_f16((uint64_t)raw[slot][p].z | ((uint64_t)raw[slot][p].w << 32));
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float16_t s = {};
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(qf[g][kk], kv[kk], s, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc += fmaxf(s[r], 0.0f) * wv[g][r];
+    }
+    // the other 16 heads of each group are in the lane 32 apart
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc), __float_as_uint(acc), false, false);
+    const float total = (__uint_as_float(sw[0]) + __uint_as_float(sw[1])) * ksc[slot];
+    const int key = 32 * (b0 + i) + j;
+    const bool live = key < lim && __builtin_amdgcn_readlane(page, i) < a.num_pages;
+    if (h == 0 && key < cols) out[key] = live ? total : fill;
+  };
+  if (live_blocks > 0) {
+#pragma unroll
+    for (int s = 0; s < kDsaAhead; ++s)
+      if (s < live_blocks) load(s, s);
+    // kDsaAhead + 1 blocks per trip, so every register slot is a constant; the trips before the last blocks test nothing
+    constexpr int S = kDsaAhead + 1;
+    int i = 0;
+    for (; i + S + kDsaAhead <= live_blocks; i += S) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        load(i + s + kDsaAhead, (s + kDsaAhead) % S);
+        compute(i + s, s);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < S + kDsaAhead - 1; ++s) {   // the rest (fewer than S + kDsaAhead blocks)
+      if (i + s + kDsaAhead < live_blocks) load(i + s + kDsaAhead, (s + kDsaAhead) % S);
+      if (i + s < live_blocks) compute(i + s, s % S);
+    }
+  }
+  for (int i = max(live_blocks, 0); i < n_blocks; ++i) {
+    const int key = 32 * (b0 + i) + j;
+    if (h == 0 && key < cols) out[key] = fill;
+  }
+}
+
 }  // namespace
 }  // namespace xt
 
@@ -923,10 +1023,29 @@ static int dsa_common(const char* what, DsaArgs& a, int dim, xt_stream_t stream)
   if (dim != 64 && dim != 128 && dim != 256) return fail(XT_EUNSUPPORTED, "%s: head size %d (64, 128, 256)", what, dim);
   if (!aligned(a.q, 8) || a.q_rs % 8 || a.q_hs % 8 || !aligned(a.w, 4) || a.ld < a.out_cols)
     return fail(XT_EINVAL, "%s: q rows must be 8-byte aligned and ld >= the columns written", what);
-  a.keys_per_wg = 4096;
-  const dim3 grid((unsigned)((a.num_q + kDsaWaves - 1) / kDsaWaves), (unsigned)((a.out_cols + 4095) / 4096));
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int nk = dim / 16, groups = a.heads / 32;
+  if (a.block > 0 && a.block % 32 == 0 && groups * nk <= 16 && aligned(a.k, 16) && a.page_bytes % 16 == 0 &&
+      a.num_q <= 65535) {
+    // blocks per wavefront: about 8 wavefronts per CU over the whole [rows, columns] area, at most 64 (one table
+    // entry per lane). Rows end early at their lengths, and the workgroups behind write the fill and leave. More
+    // wavefronts repeat the query's load and conversion (16 per CU: 22.8 us, 32: 23.3), fewer leave CUs short of loads
+    // (6: 25.9 us).
+    const int64_t blocks = ((int64_t)a.out_cols + 31) / 32;
+    const int64_t per = (blocks * a.num_q + 8 * device_cus() - 1) / (8 * device_cus());
+    const int bpw = (int)std::min<int64_t>(64, std::max<int64_t>(1, per));
+    const dim3 grid((unsigned)((blocks + (int64_t)bpw * kDsaWaves - 1) / (bpw * kDsaWaves)), (unsigned)a.num_q);
+#define XT_DSA_PAGED(NK, G)                                                                                          \
+  if (nk == NK && groups == G) {                                                                                     \
+    hipLaunchKernelGGL((dsa_paged_kernel<NK, G>), grid, dim3(64 * kDsaWaves), 0, st, a, bpw);                       \
+    return check_launch(what);                                                                                       \
+  }
+    XT_DSA_PAGED(4, 1) XT_DSA_PAGED(4, 2) XT_DSA_PAGED(4, 3) XT_DSA_PAGED(4, 4) XT_DSA_PAGED(8, 1) XT_DSA_PAGED(8, 2)
+    XT_DSA_PAGED(16, 1)
+#undef XT_DSA_PAGED
+  }
+  a.keys_per_wg = 4096;
+  const dim3 grid((unsigned)((a.num_q + kDsaWaves - 1) / kDsaWaves), (unsigned)((a.out_cols + 4095) / 4096));
   if (a.block == 0 && groups * nk <= 16 && aligned(a.k, 16) && a.k_rs % 16 == 0) {
 #define XT_DSA_FLAT(NK, G)                                                                                           \
   if (nk == NK && groups == G) {                                                                                     \
