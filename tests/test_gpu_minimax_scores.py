@@ -162,6 +162,49 @@ def test_prefill_scores(prefix, ext, dim, bs, heads, q_dtype):
             assert (err <= (bound + 2.0 ** -23 * np.abs(want[:, row, :nb]))[f]).all(), (r, t)
 
 
+@pytest.mark.parametrize('prefix,ext,dim,bs,heads,q_dtype', [
+    ([3000], [1100], 128, 32, 4, torch.bfloat16),     # enough row tiles for four column groups per wavefront
+    ([130, 1], [2100, 1997], 128, 32, 1, torch.float16),
+    ([65], [2051], 64, 32, 2, torch.bfloat16),
+])
+def test_prefill_scores_many_row_tiles(prefix, ext, dim, bs, heads, q_dtype):
+    test_prefill_scores(prefix, ext, dim, bs, heads, q_dtype)
+
+
+@pytest.mark.parametrize('dim,heads,bs,score_type,q_dtype', [
+    (128, 1, 32, 'max', torch.bfloat16), (128, 3, 64, 'lse', torch.float16), (128, 4, 256, 'max', torch.float16),
+    (128, 5, 128, 'max', torch.bfloat16), (64, 8, 128, 'lse', torch.bfloat16), (64, 7, 256, 'max', torch.bfloat16),
+    (64, 9, 64, 'max', torch.float16), (256, 2, 128, 'lse', torch.bfloat16), (256, 1, 256, 'lse', torch.float16),
+    (256, 3, 32, 'max', torch.bfloat16)])
+def test_decode_scores_few_heads(dim, heads, bs, score_type, q_dtype):
+    """Head counts at and past those whose (head, scale block) pairs fill the matrix rows, lengths at tile and block
+    edges, and slots given as s - max_slots (the reference's wrap-around)."""
+    g = torch.Generator().manual_seed(dim + heads + bs)
+    seq_lens = [1, 31, 32, 33, bs - 1, bs, bs + 1, 2100]
+    r2t, pages = _mapping(seq_lens, g, 2304)
+    pay, sc = _pool(pages, dim, g)
+    back = r2t.clone()
+    back[:, ::3] -= pages * PAGE
+    b = len(seq_lens)
+    q = (torch.randn(b, heads, dim, generator=g) * 0.5).to(q_dtype)
+    sid = torch.arange(b, dtype=torch.int32)
+    score = torch.full((heads, b, -(-2100 // bs) + 1), 7.0, device='cuda')
+    ops.minimax_decode_scores(q.cuda(), pay.cuda(), sc.cuda(), back.cuda(), score,
+                              torch.tensor(seq_lens, dtype=torch.int32).cuda(), sid.cuda(), bs, dim ** -0.5, 1.25, 1, 0,
+                              score_type)
+    got = score.cpu().numpy().astype(np.float64)
+    want = ref.minimax_block_scores_decode(q.float().numpy(), pay.numpy(), sc.numpy(), r2t.numpy(), sid.numpy(),
+                                           seq_lens, bs, dim ** -0.5, 1.25, 1, 0, score_type)
+    c, keys = ops.minimax_score_factor(dim ** -0.5, 1.25), np.abs(_keys(pay, sc))
+    for r, n in enumerate(seq_lens):
+        nb = -(-n // bs)
+        assert (got[:, r, nb:] == 7.0).all()
+        w, o = want[:, r, :nb], got[:, r, :nb]
+        bound = _block_bound(q[r].float().numpy(), keys, r2t[r].long().numpy(), n, bs, c)
+        tol = bound + 2.0 ** -23 * np.abs(w) + (4e-6 * (1 + np.abs(w)) if score_type == 'lse' else 0)
+        assert ((o == w) | (np.abs(o - w) <= tol)).all(), (r, float(np.abs(o - w).max()))
+
+
 @pytest.mark.parametrize('bs', [96, 160, 192, 224])
 def test_block_sizes_not_powers_of_two_are_refused(bs):
     """Block sizes must be 32, 64, 128 or 256 (the reference's tl.arange(0, block_size) takes powers of two): the

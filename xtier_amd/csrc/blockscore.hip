@@ -19,6 +19,8 @@
 #include "xt_common.h"
 #include "xt_host.h"
 
+#include <type_traits>
+
 namespace xt {
 namespace {
 
@@ -37,8 +39,9 @@ __device__ inline int64_t load_index(const void* p, int64_t i, bool wide) {
 }
 
 // slot -> [0, max_slots): (s + max_slots) % max_slots for the reference's range s >= -max_slots, and kept in range
-// for any other value
+// for any other value. Slots already in range skip the 64-bit division (about 100 instructions, once per key).
 __device__ inline int64_t wrap_slot(int64_t s, int64_t max_slots) {
+  if ((uint64_t)s < (uint64_t)max_slots) return s;
   const int64_t r = s % max_slots;
   return r < 0 ? r + max_slots : r;
 }
@@ -98,6 +101,24 @@ __device__ inline u32x4_t fp4x8_scaled(uint32_t w, float sf) {
     r[1] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<1>(w) * s2);
     r[2] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<2>(w) * s2);
     r[3] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<3>(w) * s2);
+  }
+  return r;
+}
+
+// The codes alone, without a scale.
+template <bool BF>
+__device__ inline u32x4_t fp4x8_plain(uint32_t w) {
+  u32x4_t r;
+  if constexpr (BF) {
+    r[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 0));
+    r[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 1));
+    r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 2));
+    r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, 1.0f, 3));
+  } else {
+    r[0] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<0>(w));
+    r[1] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<1>(w));
+    r[2] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<2>(w));
+    r[3] = __builtin_bit_cast(uint32_t, fp4x2_to_f16<3>(w));
   }
   return r;
 }
@@ -203,24 +224,160 @@ __global__ __launch_bounds__(64 * kScoreWaves) void decode_scores_kernel(const S
   }
 }
 
+// Decode for at most 32 / NK heads (4 at 128 dims): the 32 rows of the MFMA's A operand are (head, 16-dim scale block)
+// pairs, the query block-diagonal: row (head, b) holds the head's query in block b's dims and 0 elsewhere. B is the
+// unscaled key tile (one conversion per two values), and C holds, for one key per lane, the partial dot product of
+// every head and of the lane half's NK / 2 blocks, so the block scales enter as one FMA per (head, block) in FP32
+// (E4M3 values, exact). The kernel above multiplies every key value by its scale and spends its columns past `heads`
+// on nothing. Work split as above; the next block's slots are looked up behind the current block's loads. Bound: HBM, 76
+// bytes per key at 128 dims. 32 requests x 32768 keys, 4 heads: 20.8 us (3.8 TB/s) against 28.4 us for the kernel above
+// (22.1 us at 152 registers, three wavefronts per SIMD, hence the four in the launch bounds at up to 4 tiles).
+// A lane half's NK / 2 scale bytes, as loaded and as FP32.
+template <int NK>
+using ScaleWord = std::conditional_t<NK == 4, uint16_t, std::conditional_t<NK == 8, uint32_t, uint64_t>>;
+template <int NK>
+__device__ inline void key_scales(ScaleWord<NK> w, float (&f)[NK / 2]) {
+#pragma unroll
+  for (int i = 0; i < NK / 4; ++i) {
+    const half2_t v = fp8x2_to_f16<false>((uint32_t)(w >> (16 * i)));
+    f[2 * i] = (float)v[0];
+    f[2 * i + 1] = (float)v[1];
+  }
+}
+
+template <int CTRL>
+__device__ inline float dpp(float x) {   // x of the lane the DPP control names (row rotations: always a live lane)
+  return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), CTRL, 0xF, 0xF, true));
+}
+// Maximum and sum over the 32 lanes of a wavefront half (row rotations by 8, 4, 2, 1, then the row 16 apart).
+__device__ inline float half_max(float x) {
+  x = fmaxf(x, dpp<0x128>(x)); x = fmaxf(x, dpp<0x124>(x)); x = fmaxf(x, dpp<0x122>(x)); x = fmaxf(x, dpp<0x121>(x));
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+}
+__device__ inline float half_sum(float x) {
+  x += dpp<0x128>(x); x += dpp<0x124>(x); x += dpp<0x122>(x); x += dpp<0x121>(x);
+  const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+template <int NK, int T>   // wavefronts per SIMD that the registers leave
+constexpr int kFewWaves = NK <= 8 && T <= 4 ? 4 : NK * T >= 128 ? 1 : 2;
+
+template <int NK, int T, bool BF>
+__global__ __launch_bounds__(64 * kScoreWaves, (kFewWaves<NK, T>)) void decode_scores_few_kernel(const ScoreArgs a) {
+  constexpr int D = 16 * NK, NB = NK / 2, H = 16 / NB;   // scale blocks of a lane half; heads
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+  const int b = blockIdx.y;
+  const int64_t seq = load_index(a.seq_lens, b, a.wide & kWideSeq);
+  const int64_t nb = (seq + 32 * T - 1) / (32 * T);
+  if (a.skip_topk >= 0 && nb <= a.skip_topk) return;
+  int64_t blk = (int64_t)blockIdx.x * kScoreWaves + wave;
+  if (blk >= nb) return;   // no barrier below
+  const int64_t sid = wrap_slot(load_index(a.slot_ids, b, a.wide & kWideSlot), a.max_slots);
+  const int64_t r2t_row = sid * a.r2t_stride;
+  const bool wide_r2t = a.wide & kWideR2t;
+  int64_t slot[T];
+  auto load_slots = [&](int64_t at) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int64_t pos = at * (32 * T) + 32 * t + j;
+      slot[t] = pos < seq ? load_index(a.r2t, r2t_row + pos, wide_r2t) : 0;
+    }
+  };
+  load_slots(blk);
+  // A: C row 8 (r / 4) + 4 half + r % 4 (r = 0 .. 15) is head r / NB, block NB half + r % NB, so that a lane's C rows
+  // are the blocks of its own half. k-step kk covers dims h d/2 + 8 kk .. + 7 (block NB h + kk / 2) in both operands.
+  const int r_row = 4 * (j >> 3) + (j & 3), q_head = r_row / NB, q_blk = r_row % NB;
+  const bool own = ((j >> 2) & 1) == h && q_head < a.heads;
+  u32x4_t qv[NK];
+  {
+    const uint16_t* qp = a.q + (int64_t)b * a.q_ns + (int64_t)(own ? q_head : 0) * a.q_hs + h * (D / 2) + 16 * q_blk;
+    const u32x4_t q0 = *reinterpret_cast<const u32x4_t*>(qp), q1 = *reinterpret_cast<const u32x4_t*>(qp + 8);
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) qv[kk] = own && kk / 2 == q_blk ? (kk & 1 ? q1 : q0) : u32x4_t{0, 0, 0, 0};
+  }
+  const int64_t local_start = nb - a.local_blocks > 0 ? nb - a.local_blocks : 0;
+  for (; blk < nb; blk += (int64_t)gridDim.x * kScoreWaves) {
+    // every load of the block first, then the next block's slots
+    u32x4_t pw[T][NK / 4];
+    ScaleWord<NK> sw[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int64_t s = wrap_slot(slot[t], a.max_slots);
+      const uint8_t* pp = a.pay + (s >> 7) * a.pay_ps + (s & (kPoolRows - 1)) * a.pay_rs + h * (D / 4);
+      sw[t] = *reinterpret_cast<const ScaleWord<NK>*>(a.sc + (s >> 7) * a.sc_ps + (s & (kPoolRows - 1)) * a.sc_rs +
+                                                      h * (D / 32));
+#pragma unroll
+      for (int i = 0; i < NK / 4; ++i) pw[t][i] = *reinterpret_cast<const u32x4_t*>(pp + 16 * i);
+    }
+    const int64_t next = blk + (int64_t)gridDim.x * kScoreWaves;
+    if (next < nb) load_slots(next);
+    const int64_t left = seq - blk * (32 * T);   // live keys of the block
+    float v[T][H], m[H];
+#pragma unroll
+    for (int i = 0; i < H; ++i) m[i] = -__builtin_inff();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      float sc[NB];
+      key_scales<NK>(sw[t], sc);
+      float16_t s = {};
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) s = mfma16<BF>(qv[kk], fp4x8_plain<BF>(pw[t][kk / 4][kk % 4]), s);
+#pragma unroll
+      for (int i = 0; i < H; ++i) {
+        float x = s[NB * i] * sc[0];
+#pragma unroll
+        for (int k = 1; k < NB; ++k) x = __builtin_fmaf(s[NB * i + k], sc[k], x);
+        x = swap32_sum(x);
+        v[t][i] = 32 * t + j < left ? x * a.c : -__builtin_inff();
+        m[i] = fmaxf(m[i], v[t][i]);
+      }
+    }
+    float score = 0.0f;
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      float r = half_max(m[i]);
+      if (a.lse) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int t = 0; t < T; ++t) sum += exp2f(v[t][i] - r);
+        r += log2f(half_sum(sum));
+        if (r != r) r = -__builtin_inff();
+      }
+      score = j == i ? r : score;
+    }
+    if (blk >= local_start) score = 1e29f;
+    else if (blk < a.init_blocks) score = 1e30f;
+    if (lane < min(H, a.heads)) store_score(a, (int64_t)lane * a.s_hs + (int64_t)b * a.s_ns + blk * a.s_ks, score);
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
-// Prefill: grid (row tile x block range, request b, head group of HPW heads); a workgroup covers R = 256 / HPW query
+// Prefill: grid (row tile x block range, request b, head group of HPW heads); a workgroup covers R = 128 G / HPW query
 // rows of request b and one range of chunk_blocks blocks (the per-block results are independent, so ranges split a
-// long prompt's work over many workgroups). Column j of wavefront w's column group g is (row (32 / HPW)(2 w + g) + j / HPW, head j % HPW).
-// Key chunks of S = min(block_size, 128) positions are staged as 16-bit values in LDS by the whole workgroup (once
-// for its 256 columns), then each wavefront runs its two column groups over them. Chunks wholly at or below every
-// row's position skip the causal test and scale once after the maximum (c > 0: the maximum commutes with the
-// rounding of the product).
+// long prompt's work over many workgroups). Column j of wavefront w's column group g is (row (32 / HPW)(G w + g) +
+// j / HPW, head j % HPW). Key chunks of S = min(block_size, kStageKeys) positions are staged as 16-bit values in LDS
+// by the whole workgroup (two threads per key, once for its 128 G columns), then each wavefront runs its G column
+// groups over them. Two LDS stages: while one is computed on, the next chunk's payload and scales are in flight to
+// registers and the slots of the one after are being looked up, and one barrier per chunk suffices. Chunks wholly at
+// or below every row's position skip the causal test and scale once after the maximum (c > 0: the maximum commutes
+// with the rounding of the product).
+// Bound: the matrix cores, with the staging's conversions and LDS reads beside them, so G = 4 shares each staged key and
+// each LDS read among twice the columns. 4096 rows x 4 heads against 65536 keys at 128 dims (266 GFLOP): 235 us (1130
+// TFLOP/s) against 400 us for one LDS stage, G = 2 and a 64-bit division per staged piece.
 
-constexpr int kStageKeys = 128;
+template <int NK>
+constexpr int kStageKeys = NK <= 8 ? 128 : 64;
 
-template <int NK, int HPW, bool BF>
-__global__ __launch_bounds__(64 * kScoreWaves) void prefill_scores_kernel(const ScoreArgs a) {
+template <int NK, int HPW, int G, bool BF>
+__global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(const ScoreArgs a) {
   constexpr int D = 16 * NK;
   constexpr int ROW_U32 = D / 2 + 4;          // LDS row: D 16-bit values + 16 bytes of padding
-  constexpr int R = 256 / HPW;                // rows per workgroup
+  constexpr int R = 128 * G / HPW;            // rows per workgroup
   constexpr int RG = 32 / HPW;                // rows per column group
-  __shared__ uint32_t lds[kStageKeys * ROW_U32];
+  constexpr int SK = kStageKeys<NK>;
+  __shared__ uint32_t lds[2][SK * ROW_U32];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5, tid = threadIdx.x;
   const int b = blockIdx.y;
   const int64_t q0 = load_index(a.cu_seqlens, b, a.wide & kWideCu);
@@ -232,84 +389,112 @@ __global__ __launch_bounds__(64 * kScoreWaves) void prefill_scores_kernel(const 
   const int64_t pre = load_index(a.prefix_lens, b, a.wide & kWidePrefix);
   const int64_t sid = wrap_slot(load_index(a.slot_ids, b, a.wide & kWideSlot), a.max_slots);
   const int bs = a.block_size;
-  // rows of this lane's two columns, their heads and block counts
-  int64_t row[2], nblk[2];
-  bool live[2];
-  u32x4_t qv[2][NK];
-  const int head = HPW * blockIdx.z + (j % HPW);
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    row[g] = row0 + RG * (2 * wave + g) + j / HPW;
-    live[g] = row[g] < q_len && head < a.heads;
-    const int64_t hi = min(seq, pre + 64 * (row[g] / 64 + 1));
-    nblk[g] = live[g] ? (hi + bs - 1) / bs : 0;
-    const uint16_t* qp = a.q + (q0 + (live[g] ? row[g] : 0)) * a.q_ns + (int64_t)(live[g] ? head : 0) * a.q_hs +
-                         h * (D / 2);
-#pragma unroll
-    for (int kk = 0; kk < NK; ++kk)
-      qv[g][kk] = live[g] ? *reinterpret_cast<const u32x4_t*>(qp + 8 * kk) : u32x4_t{0, 0, 0, 0};
-  }
   // the workgroup's block count: that of its last live row (block counts grow with the row)
   const int64_t last = min(q_len, row0 + R) - 1;
   const int64_t wg_blocks = (min(seq, pre + 64 * (last / 64 + 1)) + bs - 1) / bs;
   const int64_t blk_lo = (int64_t)chunk * a.chunk_blocks, blk_hi = min(wg_blocks, blk_lo + a.chunk_blocks);
   if (blk_lo >= wg_blocks) return;   // uniform: before every barrier
-  const int64_t first_pos = pre + row0;       // every row of the workgroup sees keys at or below this
   const bool wide_r2t = a.wide & kWideR2t;
-  const int S = bs < kStageKeys ? bs : kStageKeys;
-  const int chunks16 = S * NK;                // 16-value pieces per stage
-  for (int64_t blk = blk_lo; blk < blk_hi; ++blk) {
-    float m[2] = {-__builtin_inff(), -__builtin_inff()};    // scaled maxima of masked chunks
-    float mr[2] = {-__builtin_inff(), -__builtin_inff()};   // raw maxima of unmasked chunks
-    for (int sub = 0; sub < bs; sub += S) {
-      const int64_t key0 = blk * bs + sub;
-      __syncthreads();   // the previous stage's readers are done
-      for (int c = tid; c < chunks16; c += 64 * kScoreWaves) {
-        const int key = c / NK, kc = c % NK;
-        const int64_t pos = key0 + key;
-        const int64_t slot =
-            pos < seq ? wrap_slot(load_index(a.r2t, sid * a.r2t_stride + pos, wide_r2t), a.max_slots) : 0;
-        const uint8_t* pp = a.pay + (slot >> 7) * a.pay_ps + (slot & (kPoolRows - 1)) * a.pay_rs + 8 * kc;
-        const uint8_t* sp = a.sc + (slot >> 7) * a.sc_ps + (slot & (kPoolRows - 1)) * a.sc_rs + kc;
-        const uint2 w = *reinterpret_cast<const uint2*>(pp);
-        const float sf = scale_of(*sp);
-        *reinterpret_cast<u32x4_t*>(&lds[key * ROW_U32 + 8 * kc]) = fp4x8_scaled<BF>(w.x, sf);
-        *reinterpret_cast<u32x4_t*>(&lds[key * ROW_U32 + 8 * kc + 4]) = fp4x8_scaled<BF>(w.y, sf);
+  const int S = bs < SK ? bs : SK;
+  const int subs = bs / S;                                // chunks per block
+  const int n_chunks = (int)(blk_hi - blk_lo) * subs;
+  const int64_t pos_lo = blk_lo * bs;                     // first position of the range
+  const int64_t r2t_row = sid * a.r2t_stride;
+  // staging: thread 2 key + half takes that half of the key's dims
+  const int s_key = tid >> 1, s_half = tid & 1;
+  const bool stager = s_key < S;
+  auto slot_at = [&](int n) -> int64_t {   // of this thread's key in chunk n; positions past the row read slot 0
+    const int64_t pos = pos_lo + (int64_t)n * S + s_key;
+    return stager && n < n_chunks && pos < seq ? load_index(a.r2t, r2t_row + pos, wide_r2t) : 0;
+  };
+  u32x4_t raw[NK / 4];
+  ScaleWord<NK> raw_sc;
+  auto load_raw = [&](int64_t slot) {
+    const int64_t s = wrap_slot(slot, a.max_slots);
+    const uint8_t* pp = a.pay + (s >> 7) * a.pay_ps + (s & (kPoolRows - 1)) * a.pay_rs + s_half * (D / 4);
+    const uint8_t* sp = a.sc + (s >> 7) * a.sc_ps + (s & (kPoolRows - 1)) * a.sc_rs + s_half * (D / 32);
+#pragma unroll
+    for (int i = 0; i < NK / 4; ++i) raw[i] = *reinterpret_cast<const u32x4_t*>(pp + 16 * i);
+    raw_sc = *reinterpret_cast<const ScaleWord<NK>*>(sp);
+  };
+  int64_t slot_next = slot_at(0);
+  // rows of this lane's columns, their block counts, and last visible position relative to pos_lo
+  int nblk[G], vis[G];
+  u32x4_t qv[G][NK];
+  const int head = HPW * blockIdx.z + (j % HPW);
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t row = row0 + RG * (G * wave + g) + j / HPW;
+    const bool live = row < q_len && head < a.heads;
+    const int64_t hi = min(seq, pre + 64 * (row / 64 + 1));
+    nblk[g] = live ? (int)(min((hi + bs - 1) / bs, blk_hi) - blk_lo) : 0;
+    vis[g] = (int)max((int64_t)-1, min(min(pre + row, seq - 1) - pos_lo, (int64_t)0x7FFFFFFF));
+    const uint16_t* qp = a.q + (q0 + (live ? row : 0)) * a.q_ns + (int64_t)(live ? head : 0) * a.q_hs + h * (D / 2);
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+      qv[g][kk] = live ? *reinterpret_cast<const u32x4_t*>(qp + 8 * kk) : u32x4_t{0, 0, 0, 0};
+  }
+  // chunks before this one are at or below every row's position and below seq_len, whole
+  const int64_t whole = a.c > 0.0f ? max((int64_t)0, min(pre + row0 + 1, seq) - pos_lo) / S : 0;
+  load_raw(slot_next);
+  slot_next = slot_at(1);
+  float m[G], mr[G];   // scaled maxima of masked chunks, raw maxima of unmasked ones
+#pragma unroll
+  for (int g = 0; g < G; ++g) m[g] = mr[g] = -__builtin_inff();
+  for (int n = 0, sub = 0, bi = 0; n < n_chunks; ++n) {
+    uint32_t* buf = lds[n & 1];
+    if (stager) {
+      uint32_t* dst = &buf[s_key * ROW_U32 + s_half * (D / 4)];
+      float scf[NK / 2];
+      key_scales<NK>(raw_sc, scf);
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk)
+        *reinterpret_cast<u32x4_t*>(dst + 4 * kk) = fp4x8_scaled<BF>(raw[kk / 4][kk % 4], scf[kk / 2]);
+    }
+    if (n + 1 < n_chunks) {
+      load_raw(slot_next);
+      slot_next = slot_at(n + 2);
+    }
+    __syncthreads();   // chunk n is staged; every wavefront is past chunk n - 1, whose buffer chunk n + 1 takes
+    const bool unmasked = n < whole;
+    for (int t = 0; t < S / 32; ++t) {
+      float16_t s[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) s[g] = float16_t{};
+      const uint32_t* kp = &buf[(32 * t + j) * ROW_U32 + h * (D / 4)];
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) {
+        const u32x4_t kv = *reinterpret_cast<const u32x4_t*>(kp + 4 * kk);
+#pragma unroll
+        for (int g = 0; g < G; ++g) s[g] = mfma16<BF>(kv, qv[g][kk], s[g]);
       }
-      __syncthreads();
-      // every key of the chunk at or below every row's position and below seq_len, and c > 0
-      const bool unmasked = key0 + S - 1 <= first_pos && key0 + S <= seq && a.c > 0.0f;
-      for (int t = 0; t < S / 32; ++t) {
-        float16_t s0 = {}, s1 = {};
-        const uint32_t* kp = &lds[(32 * t + j) * ROW_U32 + h * (D / 4)];
+      if (unmasked) {
 #pragma unroll
-        for (int kk = 0; kk < NK; ++kk) {
-          const u32x4_t kv = *reinterpret_cast<const u32x4_t*>(kp + 4 * kk);
-          s0 = mfma16<BF>(kv, qv[0][kk], s0);
-          s1 = mfma16<BF>(kv, qv[1][kk], s1);
-        }
-        if (unmasked) {
+        for (int g = 0; g < G; ++g)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            mr[0] = fmaxf(mr[0], s0[r]);
-            mr[1] = fmaxf(mr[1], s1[r]);
-          }
-        } else {
+          for (int r = 0; r < 16; ++r) mr[g] = fmaxf(mr[g], s[g][r]);
+      } else {
+        // a key counts for a row at or after it, below seq_len
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int64_t pos = key0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-            // a key counts for a row at or after it, below seq_len
-            m[0] = fmaxf(m[0], pos <= pre + row[0] && pos < seq ? s0[r] * a.c : -__builtin_inff());
-            m[1] = fmaxf(m[1], pos <= pre + row[1] && pos < seq ? s1[r] * a.c : -__builtin_inff());
-          }
+        for (int g = 0; g < G; ++g) {
+          const int lim = vis[g] - (n * S + 32 * t + 4 * h);
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            m[g] = fmaxf(m[g], 8 * (r >> 2) + (r & 3) <= lim ? s[g][r] * a.c : -__builtin_inff());
         }
       }
     }
+    if (++sub == subs) {   // the block is complete: max(round(c x)) = round(c max(x)) for c > 0
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      // max(round(c x)) = round(c max(x)) for c > 0
-      const float v = swap32_max(fmaxf(m[g], mr[g] * a.c));
-      if (h == 0 && blk < nblk[g]) store_score(a, (int64_t)head * a.s_hs + (q0 + row[g]) * a.s_ns + blk * a.s_ks, v);
+      for (int g = 0; g < G; ++g) {
+        const float v = swap32_max(fmaxf(m[g], mr[g] * a.c));
+        const int64_t row = row0 + RG * (G * wave + g) + j / HPW;
+        if (h == 0 && bi < nblk[g])
+          store_score(a, (int64_t)head * a.s_hs + (q0 + row) * a.s_ns + (blk_lo + bi) * a.s_ks, v);
+        m[g] = mr[g] = -__builtin_inff();
+      }
+      sub = 0;
+      ++bi;
     }
   }
 }
@@ -354,6 +539,16 @@ int score_common(const char* what, ScoreArgs& a, int dim, int q_dtype, const voi
 
 template <int NK, bool BF>
 int decode_dispatch(int T, const ScoreArgs& a, dim3 grid, hipStream_t st) {
+  if (a.heads <= 32 / NK) {   // the block-diagonal query fits the MFMA's rows
+    switch (T) {
+      case 1: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 1, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
+      case 2: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 2, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
+      case 4: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 4, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
+      case 8: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 8, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
+      default: return XT_EUNSUPPORTED;
+    }
+    return XT_OK;
+  }
   switch (T) {
     case 1: hipLaunchKernelGGL((decode_scores_kernel<NK, 1, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
     case 2: hipLaunchKernelGGL((decode_scores_kernel<NK, 2, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
@@ -364,14 +559,14 @@ int decode_dispatch(int T, const ScoreArgs& a, dim3 grid, hipStream_t st) {
   return XT_OK;
 }
 
-template <int NK, bool BF>
+template <int NK, int G, bool BF>
 void prefill_dispatch(int hpw, const ScoreArgs& a, dim3 grid, hipStream_t st) {
   if (hpw == 1)
-    hipLaunchKernelGGL((prefill_scores_kernel<NK, 1, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
+    hipLaunchKernelGGL((prefill_scores_kernel<NK, 1, G, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
   else if (hpw == 2)
-    hipLaunchKernelGGL((prefill_scores_kernel<NK, 2, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
+    hipLaunchKernelGGL((prefill_scores_kernel<NK, 2, G, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
   else
-    hipLaunchKernelGGL((prefill_scores_kernel<NK, 4, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
+    hipLaunchKernelGGL((prefill_scores_kernel<NK, 4, G, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
 }
 
 }  // namespace
@@ -462,22 +657,31 @@ extern "C" int xt_minimax_prefill_scores(const void* q, int64_t q_token_stride, 
   a.heads = heads;
   a.c = score_factor;
   const int hpw = heads >= 4 ? 4 : heads >= 2 ? 2 : 1;   // heads per workgroup: 256 / hpw rows each
-  const int rows = 256 / hpw;
   // block ranges: the request's blocks are at most ceil(r2t_stride / block_size) (its positions index a row of
   // req_to_token); ranges of at least 8 blocks, at most 64 ranges
   const int64_t max_blocks = (r2t_stride + block_size - 1) / block_size;
   const int64_t want_chunks = (max_blocks + 7) / 8;
   a.chunks = want_chunks < 1 ? 1 : want_chunks > 64 ? 64 : (int)want_chunks;
   a.chunk_blocks = max_blocks > 0 ? (int)((max_blocks + a.chunks - 1) / a.chunks) : 0x7FFFFFFF;
+  // four column groups per wavefront share each staged key where the query fits the registers and the row tiles
+  // still give every CU its two workgroups
+  const int64_t tiles4 = ((int64_t)max_q_len * hpw + 511) / 512;
+  const int G = dim <= 128 && tiles4 * a.chunks * batch >= 2 * device_cus() ? 4 : 2;
+  const int rows = 128 * G / hpw;
   const int64_t tiles = (max_q_len + rows - 1) / rows;
   if (tiles * a.chunks > 0x7FFFFFFF) return fail(XT_EUNSUPPORTED, "%s: %lld query tiles", what, (long long)tiles);
   const dim3 grid((unsigned)(tiles * a.chunks), (unsigned)batch, (unsigned)((heads + hpw - 1) / hpw));
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool bf = q_dtype == XT_DTYPE_BF16;
-  switch (dim) {
-    case 64: bf ? prefill_dispatch<4, true>(hpw, a, grid, st) : prefill_dispatch<4, false>(hpw, a, grid, st); break;
-    case 128: bf ? prefill_dispatch<8, true>(hpw, a, grid, st) : prefill_dispatch<8, false>(hpw, a, grid, st); break;
-    default: bf ? prefill_dispatch<16, true>(hpw, a, grid, st) : prefill_dispatch<16, false>(hpw, a, grid, st); break;
+#define XT_PREFILL(NK, G)                                                                                           \
+  bf ? prefill_dispatch<NK, G, true>(hpw, a, grid, st) : prefill_dispatch<NK, G, false>(hpw, a, grid, st)
+  if (dim == 64) {
+    if (G == 4) XT_PREFILL(4, 4); else XT_PREFILL(4, 2);
+  } else if (dim == 128) {
+    if (G == 4) XT_PREFILL(8, 4); else XT_PREFILL(8, 2);
+  } else {
+    XT_PREFILL(16, 2);
   }
+#undef XT_PREFILL
   return check_launch(what);
 }
