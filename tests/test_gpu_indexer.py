@@ -49,6 +49,21 @@ def test_topk_rows_values_placed_by_position(cols, k):
     assert np.array_equal(got, ref.topk_rows(x.numpy(), k))
 
 
+@pytest.mark.parametrize('cols', [4095, 4096, 4097, 8192, 8196, 16384, 16385, 32768, 32772, 49152, 49153, 65536, 65540,
+                                  98304, 98305])
+def test_topk_rows_edges_of_the_register_forms(cols):
+    """Rows that just fill a form and that are just past it; random, with ties at the threshold, and masked."""
+    g = torch.Generator().manual_seed(cols)
+    x = torch.randn(4, -(-cols // 4) * 4, generator=g)[:, :cols]
+    x[1] = torch.round(x[1] * 8) / 8
+    x[2, 100:cols - 700] = -math.inf
+    x[3] = 0.0
+    x[3, -5:] = 1.0
+    for k in (1, 2048):
+        got = ops.topk_rows(x.cuda(), k).cpu().numpy()
+        assert np.array_equal(got, ref.topk_rows(x.numpy(), k))
+
+
 def test_topk_rows_empty_rows():
     x = torch.randn(3, 8, device='cuda')[:, :0]          # rows of no column: nothing is read, every entry is -1
     assert np.array_equal(ops.topk_rows(x, 5).cpu().numpy(), np.full((3, 5), -1, np.int32))

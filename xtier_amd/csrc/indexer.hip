@@ -153,28 +153,29 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* x,
   for (int i = (int)k + tid; i < topk; i += kTopkThreads) o[i] = -1;
 }
 
-// Rows of at most kTopkRegCols columns (16-byte aligned rows): the row is read once into registers as order keys (a
+// Rows of at most kTopkRegMax columns (16-byte aligned rows): the row is read once into registers as order keys (a
 // non-finite value as key 0, which no finite value has; the smallest finite key is 0x00800000). Chunk i of thread t
-// holds columns 4 (kTopkRegThreads i + t) .. + 3.
+// holds columns 4 (TH i + t) .. + 3.
 //   1. A histogram of the top 13 bits finds the bucket b0 that holds the topk-th largest key (counted as the row
 //      arrives when the loads need no branches).
 //   2. One pass over the registers classifies every key: a bucket above b0 is taken (bit e of byte
-//      kTopkRegThreads i + t of the taken map, so byte j covers columns 4 j .. 4 j + 3), a key in b0 is a candidate,
+//      TH i + t of the taken map, so byte j covers columns 4 j .. 4 j + 3), a key in b0 is a candidate,
 //      appended with its column to its wavefront's list in LDS.
 //   3. Two histograms over the candidates (bits 18..9, then 8..0, both over 1024 buckets) find the topk-th largest
 //      key T and how many keys equal to T are taken; the candidates above T join the taken map, those equal to T go
 //      to the tie map. When a wavefront's list overflows, the two histograms run over the registers instead and the
 //      maps are rewritten against T.
-//   4. Thread t turns bytes 24 t .. 24 t + 23 of both maps (columns 96 t .. 96 t + 95) into positions in column
+//   4. Thread t turns bytes CH t .. CH (t + 1) - 1 of both maps (columns 4 CH t ..) into positions in column
 //      order: one block scan places them, and a key equal to T is written only while fewer than `remaining` of them
 //      come before it.
 // 1024 threads (four wavefronts per SIMD, 96 keys and 128 registers each) measured 67.5 us against 70.7 us for 512
 // threads of 192 keys on 352 rows x 95088 columns: the extra wavefronts hide more of the LDS-atomic and branch latency
-constexpr int kTopkRegThreads = 1024;
-constexpr int kTopkChunks = 24;
-constexpr int kTopkRegCols = 4 * kTopkRegThreads * kTopkChunks;   // 98304
-// one list of keys and one of columns per wavefront fill the 32 KB histogram
-constexpr int kTopkCandPerWave = 8192 / 2 / (kTopkRegThreads / 64);
+//
+// A workgroup of TH threads holds CH chunks, 4 TH CH columns, and every chunk costs its share of each pass whether the
+// row fills it or not, so a row takes the smallest form that holds it (xt_topk_rows). Measured per call at 512 keys,
+// each form against the largest: 4096 columns 8.3 us / 26.7 us (1 row), 54.4 us -> 10.0 us (352 rows, several workgroups
+// to a CU); 32768 columns 26.4 us -> 15.4 us (32 rows), 55.0 us -> 28.7 us (352 rows).
+constexpr int kTopkRegMax = 4 * 1024 * 24;   // columns of the largest form
 
 template <int NW>
 __device__ inline uint32_t block_exclusive_sum(uint32_t v, uint32_t* scratch, uint32_t& total) {
@@ -204,10 +205,10 @@ __device__ inline uint32_t block_exclusive_sum(uint32_t v, uint32_t* scratch, ui
 // in thread order is the number of keys in higher buckets. With first_topk >= 0, remaining starts as min(first_topk,
 // keys counted), returned in k. remaining is 0 afterwards when there is nothing to take (the bucket is then
 // meaningless).
-template <int NBK>
+template <int TH, int NBK>
 __device__ inline uint32_t pick_bucket(const uint32_t* h, uint32_t& remaining, uint32_t* scratch, uint32_t* sel,
                                        int first_topk = -1, uint32_t* k = nullptr) {
-  constexpr int NB = NBK / kTopkRegThreads, NW = kTopkRegThreads / 64;
+  constexpr int NB = NBK / TH, NW = TH / 64;
   const int top = NBK - 1 - NB * (int)threadIdx.x;
   uint32_t cnt[NB], sum = 0;
 #pragma unroll
@@ -246,11 +247,13 @@ __device__ inline void map_set(uint32_t* map, uint32_t col) {
 // end are masked when converted) and the loads have no branches, which lets the histogram of the first chunk rows run
 // while the later ones are still in flight. Otherwise the last chunk rows load per element behind uniform branches,
 // and the histogram starts after the whole row has arrived.
-template <bool ALIGNED4>
-__global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const float* x, int64_t ld, int cols,
+template <int TH, int CH, bool ALIGNED4>
+__global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(const float* x, int64_t ld, int cols,
                                                                           int topk, int32_t* out, int64_t out_ld) {
-  constexpr int NW = kTopkRegThreads / 64;
-  constexpr int MAPW = kTopkRegCols / 16;   // words per map
+  constexpr int NW = TH / 64;
+  constexpr int MAPW = TH * CH / 4;         // words per map
+  // one list of keys and one of columns per wavefront fill the 32 KB histogram
+  constexpr int kTopkCandPerWave = 8192 / 2 / NW;
   __shared__ __align__(16) uint32_t hist[8192];   // the 13-bit histogram, then the candidate lists
   __shared__ uint32_t hist2[1024];
   __shared__ __align__(16) uint32_t gtmap[MAPW], eqmap[MAPW];
@@ -261,22 +264,22 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
   // 1. the top 13 bits, counted as the row arrives: each chunk row's atomics run while the later chunk rows' loads
   // are still in flight, so the histogram's LDS time hides under the HBM stream
 #pragma unroll
-  for (int j = 0; j < 2048 / kTopkRegThreads; ++j)
-    reinterpret_cast<uint4*>(hist)[tid + kTopkRegThreads * j] = uint4{0, 0, 0, 0};
+  for (int j = 0; j < 2048 / TH; ++j)
+    reinterpret_cast<uint4*>(hist)[tid + TH * j] = uint4{0, 0, 0, 0};
   __syncthreads();
   // chunk row i is loaded in step i and converted and counted in step i + kTopkAhead, so kTopkAhead chunk rows of
   // loads stay in flight while the histogram's atomics run
   constexpr int kTopkAhead = 2;
-  uint32_t key[kTopkChunks][4];
+  uint32_t key[CH][4];
 #pragma unroll
-  for (int step = 0; step < kTopkChunks + kTopkAhead; ++step) {
-    if (step < kTopkChunks) {
-      const int i = step, c = 4 * (kTopkRegThreads * i + tid);
+  for (int step = 0; step < CH + kTopkAhead; ++step) {
+    if (step < CH) {
+      const int i = step, c = 4 * (TH * i + tid);
       if (ALIGNED4) {
         const float4_t v = *reinterpret_cast<const float4_t*>(xr + min(c, cols - 4));
         key[i][0] = __float_as_uint(v[0]); key[i][1] = __float_as_uint(v[1]);
         key[i][2] = __float_as_uint(v[2]); key[i][3] = __float_as_uint(v[3]);
-      } else if (4 * kTopkRegThreads * (i + 1) <= cols) {   // uniform: the whole chunk row is inside the row
+      } else if (4 * TH * (i + 1) <= cols) {   // uniform: the whole chunk row is inside the row
         const float4_t v = *reinterpret_cast<const float4_t*>(xr + c);
         key[i][0] = __float_as_uint(v[0]); key[i][1] = __float_as_uint(v[1]);
         key[i][2] = __float_as_uint(v[2]); key[i][3] = __float_as_uint(v[3]);
@@ -290,16 +293,16 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float f = __uint_as_float(key[i][e]);
-        key[i][e] = finite_f32(f) && 4 * (kTopkRegThreads * i + tid) + e < cols ? order_key(f) : 0u;
+        key[i][e] = finite_f32(f) && 4 * (TH * i + tid) + e < cols ? order_key(f) : 0u;
         if (key[i][e] != 0u) atomicAdd(&hist[key[i][e] >> 19], 1u);
       }
     }
   }
   __syncthreads();
   uint32_t remaining = 0, k = 0;
-  const uint32_t b0 = pick_bucket<8192>(hist, remaining, scratch, sel, topk, &k);
+  const uint32_t b0 = pick_bucket<TH, 8192>(hist, remaining, scratch, sel, topk, &k);
   if (k == 0) {   // uniform: no finite value
-    for (int i = tid; i < topk; i += kTopkRegThreads) o[i] = -1;
+    for (int i = tid; i < topk; i += TH) o[i] = -1;
     return;
   }
 
@@ -309,7 +312,7 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
   uint8_t* gtb = reinterpret_cast<uint8_t*>(gtmap);
   uint32_t wc = 0;
 #pragma unroll
-  for (int i = 0; i < kTopkChunks; ++i) {
+  for (int i = 0; i < CH; ++i) {
     uint32_t nib = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -322,14 +325,14 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
             wc + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
         if (c && pos < (uint32_t)kTopkCandPerWave) {
           cand_key[pos] = key[i][e];
-          cand_col[pos] = (uint32_t)(4 * (kTopkRegThreads * i + tid) + e);
+          cand_col[pos] = (uint32_t)(4 * (TH * i + tid) + e);
         }
         wc += (uint32_t)__builtin_popcountll(m);
       }
     }
-    gtb[kTopkRegThreads * i + tid] = (uint8_t)nib;
+    gtb[TH * i + tid] = (uint8_t)nib;
   }
-  for (int j = tid; j < MAPW; j += kTopkRegThreads) eqmap[j] = 0;
+  for (int j = tid; j < MAPW; j += TH) eqmap[j] = 0;
   if ((tid & 63) == 0) wcount[wave] = wc;
   __syncthreads();
   bool fits = true;
@@ -340,18 +343,18 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
   uint32_t t_key;
   if (fits) {   // uniform
     const int n = (int)wc;
-    for (int j = tid; j < 1024; j += kTopkRegThreads) hist2[j] = 0;
+    for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
     for (int j = tid & 63; j < n; j += 64) atomicAdd(&hist2[(cand_key[j] >> 9) & 1023u], 1u);
     __syncthreads();
-    const uint32_t b1 = pick_bucket<1024>(hist2, remaining, scratch, sel);
-    for (int j = tid; j < 1024; j += kTopkRegThreads) hist2[j] = 0;
+    const uint32_t b1 = pick_bucket<TH, 1024>(hist2, remaining, scratch, sel);
+    for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
     const uint32_t hi1 = (b0 << 10) | b1;
     for (int j = tid & 63; j < n; j += 64)
       if ((cand_key[j] >> 9) == hi1) atomicAdd(&hist2[cand_key[j] & 511u], 1u);
     __syncthreads();
-    const uint32_t b2 = pick_bucket<1024>(hist2, remaining, scratch, sel);
+    const uint32_t b2 = pick_bucket<TH, 1024>(hist2, remaining, scratch, sel);
     t_key = (hi1 << 9) | b2;
     for (int j = tid & 63; j < n; j += 64) {
       const uint32_t c = cand_key[j];
@@ -359,50 +362,48 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
       else if (c == t_key) map_set(eqmap, cand_col[j]);
     }
   } else {
-    for (int j = tid; j < 1024; j += kTopkRegThreads) hist2[j] = 0;
+    for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kTopkChunks; ++i)
+    for (int i = 0; i < CH; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if ((key[i][e] >> 19) == b0) atomicAdd(&hist2[(key[i][e] >> 9) & 1023u], 1u);
     __syncthreads();
-    const uint32_t b1 = pick_bucket<1024>(hist2, remaining, scratch, sel);
-    for (int j = tid; j < 1024; j += kTopkRegThreads) hist2[j] = 0;
+    const uint32_t b1 = pick_bucket<TH, 1024>(hist2, remaining, scratch, sel);
+    for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
     const uint32_t hi1 = (b0 << 10) | b1;
 #pragma unroll
-    for (int i = 0; i < kTopkChunks; ++i)
+    for (int i = 0; i < CH; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if ((key[i][e] >> 9) == hi1) atomicAdd(&hist2[key[i][e] & 511u], 1u);
     __syncthreads();
-    const uint32_t b2 = pick_bucket<1024>(hist2, remaining, scratch, sel);
+    const uint32_t b2 = pick_bucket<TH, 1024>(hist2, remaining, scratch, sel);
     t_key = (hi1 << 9) | b2;
     uint8_t* eqb = reinterpret_cast<uint8_t*>(eqmap);
 #pragma unroll
-    for (int i = 0; i < kTopkChunks; ++i) {
+    for (int i = 0; i < CH; ++i) {
       uint32_t gn = 0, en = 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         gn |= key[i][e] > t_key ? 1u << e : 0u;
         en |= key[i][e] == t_key ? 1u << e : 0u;
       }
-      gtb[kTopkRegThreads * i + tid] = (uint8_t)gn;
-      eqb[kTopkRegThreads * i + tid] = (uint8_t)en;
+      gtb[TH * i + tid] = (uint8_t)gn;
+      eqb[TH * i + tid] = (uint8_t)en;
     }
   }
   __syncthreads();
 
   // 4. positions in column order
-  constexpr int TW = MAPW / kTopkRegThreads;   // 6 words of each map per thread
+  constexpr int TW = MAPW / TH;   // words of each map per thread
   uint32_t gw[TW], ew[TW], ng = 0, ne = 0;
 #pragma unroll
-  for (int j = 0; j < TW / 2; ++j) {
-    const uint2 g = reinterpret_cast<const uint2*>(gtmap)[TW / 2 * tid + j];
-    const uint2 q = reinterpret_cast<const uint2*>(eqmap)[TW / 2 * tid + j];
-    gw[2 * j] = g.x; gw[2 * j + 1] = g.y;
-    ew[2 * j] = q.x; ew[2 * j + 1] = q.y;
+  for (int j = 0; j < TW; ++j) {
+    gw[j] = gtmap[TW * tid + j];
+    ew[j] = eqmap[TW * tid + j];
   }
 #pragma unroll
   for (int j = 0; j < TW; ++j) {
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(kTopkRegThreads) void topk_rows_reg_kernel(const fl
       }
     }
   }
-  for (int i = (int)k + tid; i < topk; i += kTopkRegThreads) o[i] = -1;
+  for (int i = (int)k + tid; i < topk; i += TH) o[i] = -1;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -914,16 +915,22 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
   if (ld < cols || out_ld < topk) return fail(XT_EINVAL, "%s: row strides shorter than the rows", what);
   // the register-resident rows read at column 0 (and at cols - 4 when cols % 4 == 0); empty rows stream, reading
   // nothing, and come out all -1
-  const bool in_registers = cols > 0 && cols <= 4 * kTopkRegThreads * kTopkChunks && ld % 4 == 0 && aligned(x, 16);
-  if (in_registers && cols % 4 == 0)
-    hipLaunchKernelGGL(topk_rows_reg_kernel<true>, dim3((unsigned)rows), dim3(kTopkRegThreads), 0,
-                       reinterpret_cast<hipStream_t>(stream), x, ld, cols, topk, out, out_ld);
-  else if (in_registers)
-    hipLaunchKernelGGL(topk_rows_reg_kernel<false>, dim3((unsigned)rows), dim3(kTopkRegThreads), 0,
-                       reinterpret_cast<hipStream_t>(stream), x, ld, cols, topk, out, out_ld);
-  else
-    hipLaunchKernelGGL(topk_rows_kernel, dim3((unsigned)rows), dim3(kTopkThreads), 0,
-                       reinterpret_cast<hipStream_t>(stream), x, ld, cols, topk, out, out_ld);
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (cols > 0 && cols <= kTopkRegMax && ld % 4 == 0 && aligned(x, 16)) {
+    const auto go = [&](auto kernel, int threads) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3((unsigned)threads), 0, st, x, ld, cols, topk, out, out_ld);
+    };
+    const bool al = cols % 4 == 0;
+#define XT_TOPK(TH, CH)                                                                                              \
+  if (cols <= 4 * TH * CH) {                                                                                         \
+    al ? go(topk_rows_reg_kernel<TH, CH, true>, TH) : go(topk_rows_reg_kernel<TH, CH, false>, TH);                   \
+    return check_launch(what);                                                                                       \
+  }
+    XT_TOPK(256, 4) XT_TOPK(512, 4) XT_TOPK(1024, 4) XT_TOPK(1024, 8) XT_TOPK(1024, 12) XT_TOPK(1024, 16)
+    XT_TOPK(1024, 24)
+#undef XT_TOPK
+  }
+  hipLaunchKernelGGL(topk_rows_kernel, dim3((unsigned)rows), dim3(kTopkThreads), 0, st, x, ld, cols, topk, out, out_ld);
   return check_launch(what);
 }
 
