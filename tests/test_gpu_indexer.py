@@ -108,6 +108,17 @@ def test_qsa_indexer_logits(rows, heads, dim, keys, dtype):
     assert (err <= bound).all(), float((err / bound).max())
 
 
+@pytest.mark.parametrize('rows,heads,dim,keys,dtype', [
+    (32, 4, 128, 63, torch.bfloat16), (33, 4, 128, 65, torch.float16), (129, 4, 128, 33000, torch.bfloat16),
+    (1, 1, 128, 1, torch.bfloat16), (300, 1, 64, 70000, torch.bfloat16), (70, 2, 256, 129, torch.float16),
+    (33, 8, 128, 64, torch.bfloat16), (40, 16, 128, 20000, torch.bfloat16), (17, 32, 256, 127, torch.float16),
+    (9, 32, 128, 31, torch.bfloat16), (2, 1, 64, (1 << 20) + 5, torch.bfloat16)])
+def test_qsa_indexer_logits_edges_of_the_tiles(rows, heads, dim, keys, dtype):
+    """Rows at and past one workgroup's for one, two and four column groups, keys at stage edges, and rows too long for
+    the 31-bit store offsets."""
+    test_qsa_indexer_logits(rows, heads, dim, keys, dtype)
+
+
 @pytest.mark.parametrize('rows,prefix', [(352, 380000), (1000, 100000), (64, 8192), (4096, 30000), (37, 500000)])
 def test_qsa_indexer_logits_reference_cases(rows, prefix):
     """The cases of tests/qsa_prefill_check.py:25-53: 4 heads x 128, compressed keys (ratio 4) up to the last row, each

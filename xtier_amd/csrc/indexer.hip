@@ -617,6 +617,170 @@ __global__ __launch_bounds__(64 * kQsaWaves) void qsa_logits_kernel(const QsaArg
   }
 }
 
+// Keys through LDS: a workgroup is 4 wavefronts x G column groups of 32 / H rows over keys_per_wg keys, S keys at a time
+// staged once for all its 128 G (row, head) columns. Queries are the MFMA rows (A: column j of a group; B: keys), so C
+// lane (key kb + j, columns 8 (r / 4) + 4 h + r % 4) holds whole rows for H <= 4 and half rows, exchanged with the lane
+// 32 apart, for H >= 8. The next stage's loads are issued before this stage's stores and the stores carry no branch
+// (rows and keys past the end have offsets past the buffer's range, which drops them), so the wait for those loads does
+// not wait for the stores behind them. The stores are non-temporal: a row's logits are read once, by the selection, and
+// are written in 512-byte pieces of 128 rows at a time (60.5 us -> 52.4 us). Bound: HBM, the FP32 logits written, with
+// the matrix product and the head sum beside it (from 8 heads on they are the larger part). 352 rows x 95088 keys, 4
+// heads x 128: 52.4 us (3.0 TB/s) against 91.8 us for the kernel above, whose wavefronts each read the keys from L2 and
+// wait for their stores with them; 352 x 65536: 8 heads 128 -> 61 us, 16 heads 261 -> 99, 32 heads 590 -> 188.
+template <int NK, int G>
+constexpr int kQsaStage = (NK <= 8 ? 64 : 32) * (G == 4 ? 2 : 1);   // keys per stage
+
+template <int H, int NK, int G, bool BF>
+__global__ __launch_bounds__(64 * kQsaWaves, 2) void qsa_logits_lds_kernel(const QsaArgs a) {
+  constexpr int D = 16 * NK, S = kQsaStage<NK, G>;
+  constexpr int ROW = D + 8;                       // 16-bit values per LDS row: conflict-free 16-byte reads
+  constexpr int kRowsG = 32 / H, kRowsW = G * kRowsG, kRowsWg = kQsaWaves * kRowsW;
+  constexpr int kPieces = S * 2 * NK / (64 * kQsaWaves);   // 16-byte pieces a thread stages
+  constexpr int kOut = H <= 4 ? 16 / H : H == 32 ? 1 : 16 / H;   // logits per lane and column group
+  __shared__ __align__(16) uint16_t lds[2][S * ROW];
+  __shared__ int2 range[kRowsWg];   // [start, end) of the rows (read behind the loop's first barrier)
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
+  const int row0 = blockIdx.x * kRowsWg, rw = row0 + wave * kRowsW;   // the workgroup's and the wavefront's first row
+  const int k_begin = blockIdx.y * a.keys_per_wg, k_end = min(a.keys, k_begin + a.keys_per_wg);
+  const int n_stages = (k_end - k_begin + S - 1) / S;
+  xt_u32x4_t raw[kPieces];
+  auto load_raw = [&](int n) {   // piece i of a thread: key (i 256 + tid) / (2 NK) of the stage
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int c = i * 64 * kQsaWaves + tid;
+      const int key = min(k_begin + n * S + c / (2 * NK), a.keys - 1);
+      raw[i] = *reinterpret_cast<const xt_u32x4_t*>(a.k + (int64_t)key * a.k_rs + 8 * (c % (2 * NK)));
+    }
+  };
+  load_raw(0);
+  for (int r = tid; r < kRowsWg; r += 64 * kQsaWaves)
+    range[r] = row0 + r < a.rows ? int2{a.starts[row0 + r], a.ends[row0 + r]} : int2{0, 0};
+  short8_t qb[G][NK];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int row = min(rw + g * kRowsG + j / H, a.rows - 1);   // rows past the end repeat the last and store nothing
+    const uint16_t* qp = a.q + (int64_t)row * a.q_rs + (int64_t)(j % H) * a.q_hs + 8 * h;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+      qb[g][kk] = __builtin_bit_cast(short8_t, *reinterpret_cast<const xt_u32x4_t*>(qp + 16 * kk));
+  }
+  // Logit (g, o) of a lane is that of row rw + g kRowsG + first(o) + h half: for H <= 4 a row's heads are H consecutive
+  // C elements of one lane, for H >= 8 the halves split pairs of rows.
+  constexpr int half = H <= 4 ? 4 / H : 1;
+  const auto first = [](int o) { return H <= 4 ? (8 * (o * H >> 2) + (o * H & 3)) / H : 2 * o; };
+  int max_start = 0, min_end = 0x7FFFFFFF, lo = 0x7FFFFFFF, hi = 0;
+  for (int r = rw + lane; r < min(rw + kRowsW, a.rows); r += 64) {
+    const int st = a.starts[r], en = a.ends[r];
+    max_start = max(max_start, st);
+    min_end = min(min_end, en);
+    lo = min(lo, max(0, st));
+    hi = max(hi, min(a.keys, en));
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    max_start = max(max_start, __shfl_xor(max_start, d));
+    min_end = min(min_end, __shfl_xor(min_end, d));
+    lo = min(lo, __shfl_xor(lo, d));
+    hi = max(hi, __shfl_xor(hi, d));
+  }
+  // uniform over the wavefront: a 32-key block outside [lo, hi) is in no row's range, one inside [max_start, min_end)
+  // in every row's
+  max_start = __builtin_amdgcn_readfirstlane(max_start);
+  min_end = __builtin_amdgcn_readfirstlane(min_end);
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  const int live_rows = min(a.rows - row0, kRowsWg);
+  float* const base = a.logits + (int64_t)row0 * a.ld;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      base, 0, (int)((int64_t)(live_rows - 1) * a.ld * 4 + (int64_t)a.keys * 4), 0x00020000);
+  const uint32_t ld4 = (uint32_t)a.ld * 4u;   // every offset of a live row is below 2^31 (host)
+  const uint32_t lane_off = (uint32_t)(wave * kRowsW + h * half) * ld4;
+  const float inv = 1.0f / a.score_scale;   // as in the kernel above
+  // the query arrives before the loop: waited for inside, its loads' counts would make every pass wait for stores
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) asm volatile("" : "+v"(qb[g][kk]));
+  for (int n = 0; n < n_stages; ++n) {
+    uint16_t* const buf = lds[n & 1];
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int c = i * 64 * kQsaWaves + tid;
+      *reinterpret_cast<xt_u32x4_t*>(buf + (c / (2 * NK)) * ROW + 8 * (c % (2 * NK))) = raw[i];
+    }
+    load_raw(min(n + 1, n_stages - 1));
+    __syncthreads();   // stage n is written; every wavefront is past stage n - 1, whose buffer stage n + 1 takes
+#pragma unroll
+    for (int t = 0; t < S / 32; ++t) {
+      const int kb = k_begin + n * S + 32 * t, key = kb + j;
+      const bool any = kb + 32 > lo && kb < hi && kb < k_end, inside = kb >= max_start && kb + 32 <= min_end;
+      const uint32_t koff = key < k_end && (H < 32 || h == 0) ? lane_off + 4u * (uint32_t)key : 0x80000000u;
+      short8_t kf[NK];
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk)
+        kf[kk] = __builtin_bit_cast(short8_t, *reinterpret_cast<const uint4*>(buf + (32 * t + j) * ROW + 16 * kk + 8 * h));
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        // formed anew for each group: kept across the loop, the store offsets would take the query's registers
+        uint32_t row_step = ld4;
+        asm volatile("" : "+s"(row_step));
+        float x[kOut];
+        if (any) {
+          float16_t sc = {};
+#pragma unroll
+          for (int kk = 0; kk < NK; ++kk) sc = mfma_qk<BF>(qb[g][kk], kf[kk], sc);
+          if constexpr (H <= 4) {
+#pragma unroll
+            for (int o = 0; o < kOut; ++o) {
+              x[o] = fmaxf(sc[o * H], 0.0f);
+#pragma unroll
+              for (int e = 1; e < H; ++e) x[o] += fmaxf(sc[o * H + e], 0.0f);
+            }
+          } else {
+            float part[32 / H];   // this half's heads of each row
+#pragma unroll
+            for (int o = 0; o < 32 / H; ++o) {
+              float quad[H / 8];
+#pragma unroll
+              for (int e = 0; e < H / 8; ++e) {
+                const int r = o * (H / 2) + 4 * e;
+                quad[e] = (fmaxf(sc[r], 0.0f) + fmaxf(sc[r + 1], 0.0f)) + (fmaxf(sc[r + 2], 0.0f) + fmaxf(sc[r + 3], 0.0f));
+              }
+              part[o] = quad[0];
+#pragma unroll
+              for (int e = 1; e < H / 8; ++e) part[o] += quad[e];
+            }
+#pragma unroll
+            for (int o = 0; o < kOut; ++o) {   // the lower half ends up with row 2 o, the upper with row 2 o + 1
+              const float p0 = part[H == 32 ? 0 : 2 * o], p1 = part[H == 32 ? 0 : 2 * o + 1];
+              const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(p0), __float_as_uint(p1), false, false);
+              x[o] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+            }
+          }
+#pragma unroll
+          for (int o = 0; o < kOut; ++o) x[o] *= inv;
+          if (!inside) {
+            // from LDS: a global load here would make the wait for the next stage's loads one for the stores as well
+            const int2* rp = range + wave * kRowsW + g * kRowsG + h * half;
+#pragma unroll
+            for (int o = 0; o < kOut; ++o) {
+              const int2 se = rp[first(o)];
+              x[o] = key >= se.x && key < se.y ? x[o] : -__builtin_inff();
+            }
+          }
+        } else {
+#pragma unroll
+          for (int o = 0; o < kOut; ++o) x[o] = -__builtin_inff();
+        }
+#pragma unroll
+        for (int o = 0; o < kOut; ++o)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[o]), rsrc, (int)(koff + (uint32_t)(g * kRowsG + first(o)) * row_step),
+                                              0, 2);
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // DSA logits (FP8)
 
@@ -948,7 +1112,7 @@ static int qsa_per_cu() {
   return n;
 }
 
-// The grid: row tiles x key chunks, the chunks sized so that the workgroups fit one round on the CUs (a second round
+// Rows too long for the LDS kernel's 31-bit offsets. The grid: row tiles x key chunks, the chunks sized so that the workgroups fit one round on the CUs (a second round
 // of a few workgroups would take as long as the first: 558 workgroups at 512 per round measured 116 us).
 template <int H, int NK, bool BF>
 static void qsa_go(QsaArgs a, int row_tiles, hipStream_t st) {
@@ -957,6 +1121,34 @@ static void qsa_go(QsaArgs a, int row_tiles, hipStream_t st) {
   a.keys_per_wg = (int)std::max<int64_t>(32, ((a.keys + chunks - 1) / chunks + 31) / 32 * 32);
   const dim3 grid((unsigned)row_tiles, (unsigned)((a.keys + a.keys_per_wg - 1) / a.keys_per_wg));
   hipLaunchKernelGGL((qsa_logits_kernel<H, NK, BF>), grid, dim3(64 * kQsaWaves), 0, st, a);
+}
+
+// As qsa_go, with the workgroups that fit a CU at two (the LDS and registers of the kernel); whole stages per chunk.
+template <int H, int NK, int G, bool BF>
+static void qsa_lds_go(QsaArgs a, hipStream_t st) {
+  constexpr int rows_wg = kQsaWaves * G * (32 / H);
+  const int tiles = (a.rows + rows_wg - 1) / rows_wg;
+  const int64_t chunks = std::max<int64_t>(1, 2 * device_cus() / tiles);
+  constexpr int S = kQsaStage<NK, G>;
+  a.keys_per_wg = (int)std::max<int64_t>(S, ((a.keys + chunks - 1) / chunks + S - 1) / S * S);
+  const dim3 grid((unsigned)tiles, (unsigned)((a.keys + a.keys_per_wg - 1) / a.keys_per_wg));
+  hipLaunchKernelGGL((qsa_logits_lds_kernel<H, NK, G, BF>), grid, dim3(64 * kQsaWaves), 0, st, a);
+}
+
+template <int H>
+static int qsa_lds_launch(int nk, bool bf, const QsaArgs& a, hipStream_t st) {
+  // the fewest column groups whose rows one workgroup holds, else as many as the registers do, except where four (and
+  // their longer stages) would leave a CU without its two workgroups
+  const int64_t wgs4 = ((int64_t)a.rows * H + 511) / 512 * ((a.keys + 127) / 128);
+#define XT_QSA(NK, G)                                                                                                \
+  if (nk == NK && (a.rows <= kQsaWaves * G * (32 / H) || G == (NK <= 8 ? 4 : 2) ||                                   \
+                   (G == 2 && wgs4 < 2 * device_cus()))) {                                                           \
+    bf ? qsa_lds_go<H, NK, G, true>(a, st) : qsa_lds_go<H, NK, G, false>(a, st);                                     \
+    return XT_OK;                                                                                                    \
+  }
+  XT_QSA(4, 1) XT_QSA(4, 2) XT_QSA(4, 4) XT_QSA(8, 1) XT_QSA(8, 2) XT_QSA(8, 4) XT_QSA(16, 1) XT_QSA(16, 2)
+#undef XT_QSA
+  return XT_EUNSUPPORTED;
 }
 
 template <int H>
@@ -1012,6 +1204,19 @@ extern "C" int xt_qsa_indexer_logits(const void* q, int64_t q_row_stride, int64_
   const bool bf = dtype == XT_DTYPE_BF16;
   const int nk = dim / 16;
   int e = XT_EUNSUPPORTED;
+  // the LDS kernel's store offsets are 31-bit: its rows per workgroup (512 / heads, 256 / heads at 256 dims) times ld
+  if ((int64_t)(512 / heads) * ld * 4 + 4 * (int64_t)keys < 0x7FFFFFFF) {
+    switch (heads) {
+      case 1: e = qsa_lds_launch<1>(nk, bf, a, st); break;
+      case 2: e = qsa_lds_launch<2>(nk, bf, a, st); break;
+      case 4: e = qsa_lds_launch<4>(nk, bf, a, st); break;
+      case 8: e = qsa_lds_launch<8>(nk, bf, a, st); break;
+      case 16: e = qsa_lds_launch<16>(nk, bf, a, st); break;
+      case 32: e = qsa_lds_launch<32>(nk, bf, a, st); break;
+    }
+    if (e != XT_OK) return fail(e, "%s: no kernel for %d heads x %d", what, heads, dim);
+    return check_launch(what);
+  }
   switch (heads) {
     case 1: e = qsa_launch<1>(nk, bf, a, row_tiles, st); break;
     case 2: e = qsa_launch<2>(nk, bf, a, row_tiles, st); break;
