@@ -186,6 +186,20 @@ def test_mla_fewer_heads(heads):
     _check(out, lse, ref, ref_lse)
 
 
+@pytest.mark.parametrize('heads,splits', [(17, 1), (112, 2), (113, 1), (128, 3)])
+def test_mla_absent_heads_and_steps_without_keys(heads, splits):
+    """Waves without a live head and 32-key steps without a valid key: first, in the middle, past a row's length."""
+    w, inp = _case(31 + heads, heads=heads)
+    pool = _pool(w, 6)
+    idx = inp.slots.clone()
+    idx[0, :64] = -1
+    idx[1, 32:256] = -1
+    lens = torch.tensor([300, 300, 1, 33, 160], dtype=torch.int32, device='cuda')
+    out, lse = ops.sparse_mla(inp.q, pool, idx, lens, None, 0.05, splits=splits)
+    ref, ref_lse = _ref(inp.q, pool, idx, lens, None, 0.05)
+    _check(out, lse, ref, ref_lse, bf16_slack=True)   # row 2 is one key's latent, rounded to BF16
+
+
 @pytest.mark.parametrize('heads,splits', [(128, 8), (128, 10), (100, 9), (16, 4), (64, 3)])
 def test_mla_split_merge_head_and_split_counts(heads, splits):
     """Key splits with head counts that pad the last 16-head wave, more splits than 16-head waves, and splits that
