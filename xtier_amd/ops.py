@@ -6,6 +6,7 @@ xtier/backend/formats.py). Tensors are torch tensors on the GPU; every call runs
 (k_pay u8 [slots, kv_heads, dim/2], v_pay, k_scales u8 [slots, kv_heads, dim/16], v_scales, gk f32 [1], gv f32 [1]).
 """
 import ctypes
+import functools
 import math
 import warnings
 
@@ -24,7 +25,9 @@ def _ptr(t):
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if t.is_cuda:
+        return torch._C._cuda_getCurrentRawStream(t.get_device())   # as below, without building the stream object
+    return torch.cuda.current_stream(t.device).cuda_stream          # raises
 
 
 def _need_cuda(*tensors):
@@ -63,10 +66,11 @@ def _check_raw(raw, contiguous=True):
     if contiguous:
         packed = k.is_contiguous() and v.is_contiguous() and k_sf.is_contiguous() and v_sf.is_contiguous()
     else:
-        packed = (all(t.dim() == 3 and t.stride(2) == 1 and (t.shape[1] == 1 or t.stride(1) >= t.shape[2])
-                      for t in (k, v, k_sf, v_sf))
-                  and k.stride()[:2] == v.stride()[:2] and k_sf.stride()[:2] == v_sf.stride()[:2]
-                  and k.shape == v.shape and k_sf.shape == v_sf.shape and k_sf.shape[2] * 8 == k.shape[2])
+        shape, stride, sf_shape, sf_stride = k.shape, k.stride(), k_sf.shape, k_sf.stride()
+        packed = (len(shape) == 3 and len(sf_shape) == 3 and v.shape == shape and v_sf.shape == sf_shape
+                  and v.stride() == stride and v_sf.stride() == sf_stride and stride[2] == 1 and sf_stride[2] == 1
+                  and (shape[1] == 1 or stride[1] >= shape[2]) and (sf_shape[1] == 1 or sf_stride[1] >= sf_shape[2])
+                  and sf_shape[2] * 8 == shape[2])
     if not (packed and dim % 32 == 0 and dim & (dim - 1) == 0):
         raise ValueError(f'xtier qsa_fp4: packed [m, heads, dim / 2] rows with a power-of-2 head size expected, got '
                          f'{tuple(k.shape)}')
@@ -294,6 +298,10 @@ _cu_counts = {}
 
 def device_cus(device=None):
     """Compute units of the current (or given) GPU, 256 on an MI355X; 256 when no GPU is visible."""
+    if device is None and _cu_counts:   # a GPU has been seen: no availability query on each call
+        n = _cu_counts.get(torch.cuda.current_device())
+        if n is not None:
+            return n
     if not torch.cuda.is_available():
         return 256
     idx = torch.cuda.current_device() if device is None else torch.device(device).index
@@ -338,6 +346,7 @@ def varlen_splits(rows, kv_heads, group, max_k):
     return default_splits(rows, kv_heads, max_k, False)
 
 
+@functools.lru_cache(maxsize=1024)   # a pure function of the sizes
 def decode_workspace_bytes(rows, q_heads, dim, splits):
     return int(_lib.lib().xt_sparse_decode_workspace_bytes(rows, q_heads, dim, splits))
 
@@ -368,11 +377,14 @@ def sparse_decode(q, raw, table, indices, seq_lens, scale, page_size=1, row_req=
         row_req = row_req.to(torch.int64)
     seq_lens, counts, query_pos = (None if t is None else (t if t.dtype == torch.int32 else t.to(torch.int32))
                                    for t in (seq_lens, counts, query_pos))
-    args = (_ptr(q), q.stride(0), q.stride(1), *map(_ptr, raw), raw[0].shape[0], raw[0].stride(0), raw[2].stride(0),
-            _head_stride(raw[0]), _head_stride(raw[2]), kv_heads, q_heads, dim, _ptr(table), table.stride(0),
-            int(page_size), _ptr(row_req), _ptr(indices), indices.stride(0), topk, _ptr(counts), _ptr(seq_lens),
-            _ptr(query_pos), float(scale), _ptr(out), out.stride(0), out.stride(1), _DTYPES[out.dtype], _ptr(lse),
-            rows)
+    k, v, k_sf, v_sf, gk, gv = raw
+    q_stride, out_stride, pay_stride, sf_stride = q.stride(), out.stride(), k.stride(), k_sf.stride()
+    args = (q.data_ptr(), q_stride[0], q_stride[1], k.data_ptr(), v.data_ptr(), k_sf.data_ptr(), v_sf.data_ptr(),
+            gk.data_ptr(), gv.data_ptr(), k.shape[0], pay_stride[0], sf_stride[0],
+            pay_stride[1] if kv_heads > 1 else 0, sf_stride[1] if kv_heads > 1 else 0, kv_heads, q_heads, dim,
+            table.data_ptr(), table.stride(0), int(page_size), _ptr(row_req), indices.data_ptr(), indices.stride(0),
+            topk, _ptr(counts), _ptr(seq_lens), _ptr(query_pos), float(scale), out.data_ptr(), out_stride[0],
+            out_stride[1], _DTYPES[out.dtype], _ptr(lse), rows)
     if isinstance(ws, str) and ws == 'static':
         # the library's own per-GPU scratch array: nothing is allocated for this call
         splits = default_splits(rows, kv_heads, topk) if splits is None else splits
@@ -404,18 +416,19 @@ _warned = set()
 def _capture_splits(device, rows, q_heads, dim, splits, ws):
     """``splits``, or 1 inside a graph capture whose cached workspace is too small (one key split needs no partials,
     so no workspace has to grow inside the capture), with a warning."""
-    need = decode_workspace_bytes(rows, q_heads, dim, splits)
-    if splits > 1 and ws is None and torch.cuda.is_current_stream_capturing() and _cached_workspace_bytes(device) < need:
-        return _narrowed('sparse_decode', splits, 1, need)
+    if splits > 1 and ws is None:
+        need = decode_workspace_bytes(rows, q_heads, dim, splits)
+        if _cached_workspace_bytes(device) < need and torch.cuda.is_current_stream_capturing():
+            return _narrowed('sparse_decode', splits, 1, need)
     return splits
 
 
 def _decode_ws(device, rows, q_heads, dim, splits, ws):
     """The caller's workspace, else the per-device one (a throwaway buffer for one split inside a capture that the
     cached one cannot serve: the kernel never reads it then)."""
-    need = decode_workspace_bytes(rows, q_heads, dim, splits)
     if ws is not None:
         return ws
+    need = decode_workspace_bytes(rows, q_heads, dim, splits)
     if _cached_workspace_bytes(device) >= need or not torch.cuda.is_current_stream_capturing():
         return workspace(device, need)
     return torch.empty(need, dtype=torch.uint8, device=device)
