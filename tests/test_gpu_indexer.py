@@ -64,6 +64,25 @@ def test_topk_rows_edges_of_the_register_forms(cols):
         assert np.array_equal(got, ref.topk_rows(x.numpy(), k))
 
 
+@pytest.mark.parametrize('rows,cols', [(300, 65540), (300, 20000), (270, 32768), (270, 49152), (300, 65533), (260, 98304), (257, 70001), (3, 98308), (2, 196608), (2, 196609),
+                                       (2, 150003)])
+def test_topk_rows_packed_forms(rows, cols):
+    """More rows than CUs and rows past 98304 columns keep 16 bits per key: values that differ below those bits, ties
+    that overflow the candidate lists, masked and non-finite columns."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn(rows, -(-cols // 4) * 4, generator=g)[:, :cols]
+    n = min(rows, 5)
+    x[0] = 1.0 + torch.randint(0, 1 << 15, (cols,), generator=g) * 2.0 ** -23   # one bucket, differing low bits
+    x[1] = torch.round(x[1] * 2) / 2
+    if rows > 2:
+        x[2, 5:cols - 900] = -math.inf
+        x[-1, ::3] = math.nan
+    for k in (1, 2048):
+        got = ops.topk_rows(x.cuda(), k).cpu().numpy()
+        for r in {0, 1, *range(n), rows - 1}:
+            assert np.array_equal(got[r:r + 1], ref.topk_rows(x[r:r + 1].numpy(), k)), r
+
+
 def test_topk_rows_empty_rows():
     x = torch.randn(3, 8, device='cuda')[:, :0]          # rows of no column: nothing is read, every entry is -1
     assert np.array_equal(ops.topk_rows(x, 5).cpu().numpy(), np.full((3, 5), -1, np.int32))

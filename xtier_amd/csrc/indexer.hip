@@ -14,7 +14,7 @@
 //     the paged cache (page = block x D E4M3 values, then block FP32 scales) through the block table.
 //   Top-k rows: per row the positions of the topk largest finite values, ascending (ties toward the lower position),
 //     -1 padded. One workgroup per row: a three-pass radix select over an order-preserving key finds the topk-th
-//     largest key T and how many keys equal to T are taken. Rows up to 98304 columns live in registers: the first
+//     largest key T and how many keys equal to T are taken. Rows up to 196608 columns live in registers: the first
 //     pass (13 bits) leaves a small candidate bucket whose keys go to LDS for the other two passes, and bitmaps of the
 //     taken columns are turned into positions with one block scan. Longer rows are streamed three times (11, 11, 10
 //     bits), and one pass in position order writes the positions, each 1024-position chunk placed by a block-wide
@@ -173,9 +173,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* x,
 //
 // A workgroup of TH threads holds CH chunks, 4 TH CH columns, and every chunk costs its share of each pass whether the
 // row fills it or not, so a row takes the smallest form that holds it (xt_topk_rows). Measured per call at 512 keys,
-// each form against the largest: 4096 columns 8.3 us / 26.7 us (1 row), 54.4 us -> 10.0 us (352 rows, several workgroups
-// to a CU); 32768 columns 26.4 us -> 15.4 us (32 rows), 55.0 us -> 28.7 us (352 rows).
-constexpr int kTopkRegMax = 4 * 1024 * 24;   // columns of the largest form
+// the form of 98304 columns -> the smallest: 4096 columns 26.7 us -> 8.3 us (1 row), 54.4 us -> 10.0 us (352 rows,
+// several workgroups to a CU); 32768 columns 26.4 us -> 15.4 us (32 rows).
+constexpr int kTopkRegMax = 4 * 1024 * 48;   // columns of the largest form
 
 template <int NW>
 __device__ inline uint32_t block_exclusive_sum(uint32_t v, uint32_t* scratch, uint32_t& total) {
@@ -237,17 +237,23 @@ __device__ inline uint32_t pick_bucket(const uint32_t* h, uint32_t& remaining, u
   return bucket;
 }
 
-// Sets the bit of column `col` in a byte map (byte col / 4, bit col % 4) with a word-wide LDS atomic.
-__device__ inline void map_set(uint32_t* map, uint32_t col) {
+// Sets the bit of column `col` (plus `shift`: 4 for the ties) in the byte map (byte col / 4) with a word-wide LDS atomic.
+__device__ inline void map_set(uint32_t* map, uint32_t col, uint32_t shift) {
   const uint32_t byte = col >> 2;
-  atomicOr(&map[byte >> 2], 1u << (8u * (byte & 3u) + (col & 3u)));
+  atomicOr(&map[byte >> 2], 1u << (8u * (byte & 3u) + (col & 3u) + shift));
 }
 
 // ALIGNED4: cols % 4 == 0, so every chunk row loads as float4 from an address clamped into the row (columns past the
 // end are masked when converted) and the loads have no branches, which lets the histogram of the first chunk rows run
 // while the later ones are still in flight. Otherwise the last chunk rows load per element behind uniform branches,
 // and the histogram starts after the whole row has arrived.
-template <int TH, int CH, bool ALIGNED4>
+// PACK: only the top 16 bits of a key stay in registers, two keys to one, so a CU holds two rows of 98304 columns (one
+// loads while the other computes) or one of 196608; the candidates' keys are read from the row again, and a list
+// overflow reads the row for each of its three passes. 352 rows x 95088 columns: 49.3 us (2.7 TB/s) against 63.4 us for
+// one row of whole keys per CU, 49000 columns 26.2 us against 35.1 us; 32 rows x 131072 columns 40.6 us against 205.7 us
+// for the streaming kernel. Up to one row per CU the whole keys are faster (more wavefronts per row: 26.7 us at 95088
+// columns), past it two rows to a CU are (270 rows: 42.5 us against 55.7 us).
+template <int TH, int CH, bool ALIGNED4, bool PACK>
 __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(const float* x, int64_t ld, int cols,
                                                                           int topk, int32_t* out, int64_t out_ld) {
   constexpr int NW = TH / 64;
@@ -256,7 +262,7 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
   constexpr int kTopkCandPerWave = 8192 / 2 / NW;
   __shared__ __align__(16) uint32_t hist[8192];   // the 13-bit histogram, then the candidate lists
   __shared__ uint32_t hist2[1024];
-  __shared__ __align__(16) uint32_t gtmap[MAPW], eqmap[MAPW];
+  __shared__ __align__(16) uint32_t map[MAPW];   // per byte: bits 0-3 the taken columns, bits 4-7 the ties
   __shared__ uint32_t scratch[NW], sel[2], wcount[NW];
   const int tid = threadIdx.x, wave = tid >> 6;
   const float* xr = x + (int64_t)blockIdx.x * ld;
@@ -270,34 +276,46 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
   // chunk row i is loaded in step i and converted and counted in step i + kTopkAhead, so kTopkAhead chunk rows of
   // loads stay in flight while the histogram's atomics run
   constexpr int kTopkAhead = 2;
-  uint32_t key[CH][4];
+  uint32_t key[CH][PACK ? 2 : 4];   // PACK: the top halves of elements 0, 1 and 2, 3
+  uint32_t in[kTopkAhead + 1][4];   // the chunk rows in flight
+  const auto load = [&](int i, uint32_t (&v4)[4]) {   // chunk i of the row, as bits
+    const int c = 4 * (TH * i + tid);
+    if (ALIGNED4 || 4 * TH * (i + 1) <= cols) {   // uniform: the whole chunk row is inside the row, or clamped into it
+      const float4_t v = *reinterpret_cast<const float4_t*>(xr + (ALIGNED4 ? min(c, cols - 4) : c));
+      v4[0] = __float_as_uint(v[0]); v4[1] = __float_as_uint(v[1]);
+      v4[2] = __float_as_uint(v[2]); v4[3] = __float_as_uint(v[3]);
+    } else {   // an address inside the row; columns past the end are masked when converted
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v4[e] = __float_as_uint(xr[min(c + e, cols - 1)]);
+    }
+  };
+  const auto convert = [&](int i, int e, uint32_t bits) {
+    const float f = __uint_as_float(bits);
+    return finite_f32(f) && 4 * (TH * i + tid) + e < cols ? order_key(f) : 0u;
+  };
 #pragma unroll
   for (int step = 0; step < CH + kTopkAhead; ++step) {
-    if (step < CH) {
-      const int i = step, c = 4 * (TH * i + tid);
-      if (ALIGNED4) {
-        const float4_t v = *reinterpret_cast<const float4_t*>(xr + min(c, cols - 4));
-        key[i][0] = __float_as_uint(v[0]); key[i][1] = __float_as_uint(v[1]);
-        key[i][2] = __float_as_uint(v[2]); key[i][3] = __float_as_uint(v[3]);
-      } else if (4 * TH * (i + 1) <= cols) {   // uniform: the whole chunk row is inside the row
-        const float4_t v = *reinterpret_cast<const float4_t*>(xr + c);
-        key[i][0] = __float_as_uint(v[0]); key[i][1] = __float_as_uint(v[1]);
-        key[i][2] = __float_as_uint(v[2]); key[i][3] = __float_as_uint(v[3]);
-      } else {   // an address inside the row; columns past the end are masked when converted
-#pragma unroll
-        for (int e = 0; e < 4; ++e) key[i][e] = __float_as_uint(xr[min(c + e, cols - 1)]);
-      }
-    }
+    if (step < CH) load(step, in[step % (kTopkAhead + 1)]);
     if (step >= kTopkAhead) {
       const int i = step - kTopkAhead;
+      uint32_t k4[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float f = __uint_as_float(key[i][e]);
-        key[i][e] = finite_f32(f) && 4 * (TH * i + tid) + e < cols ? order_key(f) : 0u;
-        if (key[i][e] != 0u) atomicAdd(&hist[key[i][e] >> 19], 1u);
+        k4[e] = convert(i, e, in[i % (kTopkAhead + 1)][e]);
+        if (k4[e] != 0u) atomicAdd(&hist[k4[e] >> 19], 1u);
+        if constexpr (!PACK) key[i][e] = k4[e];
+      }
+      if constexpr (PACK) {
+        key[i][0] = __builtin_amdgcn_perm(k4[1], k4[0], 0x07060302u);
+        key[i][1] = __builtin_amdgcn_perm(k4[3], k4[2], 0x07060302u);
+        asm volatile("" : "+v"(key[i][0]), "+v"(key[i][1]));   // packed here: sunk to their uses, the four keys would stay
       }
     }
   }
+  const auto bucket_of = [&](int i, int e) {   // the top 13 bits
+    if constexpr (PACK) return e & 1 ? key[i][e >> 1] >> 19 : (key[i][e >> 1] & 0xFFFFu) >> 3;
+    else return key[i][e] >> 19;
+  };
   __syncthreads();
   uint32_t remaining = 0, k = 0;
   const uint32_t b0 = pick_bucket<TH, 8192>(hist, remaining, scratch, sel, topk, &k);
@@ -309,14 +327,14 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
   // 2. classify: buckets above b0 taken, b0 appended to the wavefront's candidate list (the count stays uniform)
   uint32_t* cand_key = hist + wave * kTopkCandPerWave;
   uint32_t* cand_col = hist + (NW + wave) * kTopkCandPerWave;
-  uint8_t* gtb = reinterpret_cast<uint8_t*>(gtmap);
+  uint8_t* mapb = reinterpret_cast<uint8_t*>(map);
   uint32_t wc = 0;
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     uint32_t nib = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint32_t d = key[i][e] >> 19;
+      const uint32_t d = bucket_of(i, e);
       nib |= d > b0 ? 1u << e : 0u;
       const bool c = d == b0;
       const uint64_t m = __builtin_amdgcn_ballot_w64(c);
@@ -324,15 +342,14 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
         const uint32_t pos =
             wc + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
         if (c && pos < (uint32_t)kTopkCandPerWave) {
-          cand_key[pos] = key[i][e];
+          if constexpr (!PACK) cand_key[pos] = key[i][e];
           cand_col[pos] = (uint32_t)(4 * (TH * i + tid) + e);
         }
         wc += (uint32_t)__builtin_popcountll(m);
       }
     }
-    gtb[TH * i + tid] = (uint8_t)nib;
+    mapb[TH * i + tid] = (uint8_t)nib;
   }
-  for (int j = tid; j < MAPW; j += TH) eqmap[j] = 0;
   if ((tid & 63) == 0) wcount[wave] = wc;
   __syncthreads();
   bool fits = true;
@@ -343,6 +360,8 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
   uint32_t t_key;
   if (fits) {   // uniform
     const int n = (int)wc;
+    if constexpr (PACK)
+      for (int j = tid & 63; j < n; j += 64) cand_key[j] = order_key(xr[cand_col[j]]);
     for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
     for (int j = tid & 63; j < n; j += 64) atomicAdd(&hist2[(cand_key[j] >> 9) & 1023u], 1u);
@@ -358,42 +377,52 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
     t_key = (hi1 << 9) | b2;
     for (int j = tid & 63; j < n; j += 64) {
       const uint32_t c = cand_key[j];
-      if (c > t_key) map_set(gtmap, cand_col[j]);
-      else if (c == t_key) map_set(eqmap, cand_col[j]);
+      if (c > t_key) map_set(map, cand_col[j], 0u);
+      else if (c == t_key) map_set(map, cand_col[j], 4u);
     }
   } else {
+    // f(i, the whole keys of chunk i): from the registers, or (PACK, not unrolled) from the row again
+    const auto for_chunks = [&](auto f) {
+      if constexpr (PACK) {
+#pragma unroll 1
+        for (int i = 0; i < CH; ++i) {
+          uint32_t k4[4];
+          load(i, k4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) k4[e] = convert(i, e, k4[e]);
+          f(i, k4);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) f(i, key[i]);
+      }
+    };
     for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < CH; ++i)
+    for_chunks([&](int, const uint32_t* k4) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if ((key[i][e] >> 19) == b0) atomicAdd(&hist2[(key[i][e] >> 9) & 1023u], 1u);
+        if ((k4[e] >> 19) == b0) atomicAdd(&hist2[(k4[e] >> 9) & 1023u], 1u);
+    });
     __syncthreads();
     const uint32_t b1 = pick_bucket<TH, 1024>(hist2, remaining, scratch, sel);
     for (int j = tid; j < 1024; j += TH) hist2[j] = 0;
     __syncthreads();
     const uint32_t hi1 = (b0 << 10) | b1;
-#pragma unroll
-    for (int i = 0; i < CH; ++i)
+    for_chunks([&](int, const uint32_t* k4) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if ((key[i][e] >> 9) == hi1) atomicAdd(&hist2[key[i][e] & 511u], 1u);
+        if ((k4[e] >> 9) == hi1) atomicAdd(&hist2[k4[e] & 511u], 1u);
+    });
     __syncthreads();
     const uint32_t b2 = pick_bucket<TH, 1024>(hist2, remaining, scratch, sel);
     t_key = (hi1 << 9) | b2;
-    uint8_t* eqb = reinterpret_cast<uint8_t*>(eqmap);
+    for_chunks([&](int i, const uint32_t* k4) {
+      uint32_t n = 0;
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      uint32_t gn = 0, en = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        gn |= key[i][e] > t_key ? 1u << e : 0u;
-        en |= key[i][e] == t_key ? 1u << e : 0u;
-      }
-      gtb[TH * i + tid] = (uint8_t)gn;
-      eqb[TH * i + tid] = (uint8_t)en;
-    }
+      for (int e = 0; e < 4; ++e) n |= k4[e] > t_key ? 1u << e : k4[e] == t_key ? 16u << e : 0u;
+      mapb[TH * i + tid] = (uint8_t)n;
+    });
   }
   __syncthreads();
 
@@ -402,8 +431,9 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
   uint32_t gw[TW], ew[TW], ng = 0, ne = 0;
 #pragma unroll
   for (int j = 0; j < TW; ++j) {
-    gw[j] = gtmap[TW * tid + j];
-    ew[j] = eqmap[TW * tid + j];
+    const uint32_t w = map[TW * tid + j];
+    gw[j] = w & 0x0F0F0F0Fu;
+    ew[j] = (w >> 4) & 0x0F0F0F0Fu;
   }
 #pragma unroll
   for (int j = 0; j < TW; ++j) {
@@ -1085,13 +1115,16 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
       hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3((unsigned)threads), 0, st, x, ld, cols, topk, out, out_ld);
     };
     const bool al = cols % 4 == 0;
-#define XT_TOPK(TH, CH)                                                                                              \
-  if (cols <= 4 * TH * CH) {                                                                                         \
-    al ? go(topk_rows_reg_kernel<TH, CH, true>, TH) : go(topk_rows_reg_kernel<TH, CH, false>, TH);                   \
+    const bool many = rows > device_cus();   // past one round at one workgroup per CU: two packed ones share a CU
+#define XT_TOPK(TH, CH, PACK, RULE)                                                                                  \
+  if (cols <= 4 * TH * CH && (RULE)) {                                                                               \
+    al ? go(topk_rows_reg_kernel<TH, CH, true, PACK>, TH) : go(topk_rows_reg_kernel<TH, CH, false, PACK>, TH);       \
     return check_launch(what);                                                                                       \
   }
-    XT_TOPK(256, 4) XT_TOPK(512, 4) XT_TOPK(1024, 4) XT_TOPK(1024, 8) XT_TOPK(1024, 12) XT_TOPK(1024, 16)
-    XT_TOPK(1024, 24)
+    XT_TOPK(256, 4, false, true) XT_TOPK(512, 4, false, true) XT_TOPK(1024, 4, false, true)
+    XT_TOPK(512, 16, true, many) XT_TOPK(1024, 8, false, true) XT_TOPK(512, 24, true, many) XT_TOPK(1024, 12, false, true)
+    XT_TOPK(512, 32, true, many) XT_TOPK(1024, 16, false, true) XT_TOPK(512, 48, true, many)
+    XT_TOPK(1024, 24, false, true) XT_TOPK(1024, 48, true, true)
 #undef XT_TOPK
   }
   hipLaunchKernelGGL(topk_rows_kernel, dim3((unsigned)rows), dim3(kTopkThreads), 0, st, x, ld, cols, topk, out, out_ld);
