@@ -87,6 +87,31 @@ def test_minimax_prefill_against_oracle(bq, splits):
     check(out, ref, flash)
 
 
+@pytest.mark.parametrize('batch,bq,given,wide', [(1, 1, False, 0), (3, 64, False, 1), (5, 7, True, 2), (64, 3, False, 3),
+                                                 (65, 3, False, 0), (130, 16, True, 1)])
+def test_row_arguments(batch, bq, given, wide):
+    """The per-row arguments against their plain formula: empty requests, slots that wrap, table and list bounds, int32
+    and int64 arrays, the walk (up to 64 requests) and the search."""
+    g = torch.Generator().manual_seed(batch + bq)
+    n = torch.randint(0, 40, (batch,), generator=g) * (torch.rand(batch, generator=g) > 0.3)
+    n[-1] = 33
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), n.cumsum(0)])
+    sid = torch.randint(-256, 256, (batch,), generator=g)
+    pre, seq = torch.randint(0, 5000, (batch,), generator=g), torch.randint(0, 9000, (batch,), generator=g)
+    blk = torch.cat([torch.zeros(1, dtype=torch.int64), ((n + bq - 1) // bq).cumsum(0)])
+    total, slots, lists = int(cu[-1]), 256, int(blk[-1]) - 1
+    r2t = torch.empty(100, 6000, dtype=torch.int32)
+    dt = [torch.int64 if wide >> i & 1 else torch.int32 for i in range(2)]
+    got = ops._block_prefill_rows(cu.to(dt[0]).cuda(), sid.to(dt[1]).cuda(), pre.to(dt[1]).cuda(), seq.to(dt[0]).cuda(),
+                                  blk.int().cuda() if given else None, total, bq, slots, r2t, max(1, lists))
+    b = torch.repeat_interleave(torch.arange(batch), n)
+    local = torch.arange(total) - cu[b]
+    want = ((sid[b] % slots).clamp(max=99), seq[b].clamp(max=6000), pre[b] + local,
+            (blk[b] + local // bq).clamp(max=max(1, lists) - 1))
+    for x, y in zip(got, want):
+        assert torch.equal(x.cpu().long(), y)
+
+
 def test_strided_pool_kv_scale_and_queries_without_keys():
     print('block-sparse prefill: strided pool, kv_scale, empty rows', flush=True)
     c = _case(77, q_lens=(40, 70), prefix=(300, 129), bq=16, topk=3)

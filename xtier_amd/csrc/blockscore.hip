@@ -499,6 +499,56 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
   }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// The per-row arguments of a ragged block-sparse prefill (kv_fp4.py:384-400 derives them per program): thread = row.
+
+struct RowArgs {
+  const void *cu_seqlens, *slot_ids, *prefix_lens, *seq_lens;   // [batch + 1], [batch] ...
+  const int64_t* cu_blocks;   // [batch + 1] query blocks before each request, or NULL: from cu_seqlens
+  int wide;
+  int batch, rows, block_q;
+  int64_t max_slots;
+  int reqs, width, list_rows;   // req_to_token rows and columns, list rows: upper bounds
+  int64_t* row_req;
+  int32_t *row_seq, *row_qpos, *row_idx;
+};
+
+__global__ __launch_bounds__(256) void prefill_rows_kernel(const RowArgs a) {
+  const int r = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (r >= a.rows) return;
+  const bool wide_cu = a.wide & kWideCu;
+  // the request: how many of cu[1:] are at or below r; without cu_blocks the walk counts the blocks on its way
+  int b = 0;
+  int64_t start = load_index(a.cu_seqlens, 0, wide_cu), blocks = 0;
+  if (a.cu_blocks) {
+    int n = a.batch - 1;   // of cu[1 .. batch - 1]: the last request takes every row left
+    while (n > 0) {
+      const int half = n / 2;
+      if (load_index(a.cu_seqlens, b + half + 1, wide_cu) <= r) {
+        b += half + 1;
+        n -= half + 1;
+      } else {
+        n = half;
+      }
+    }
+    start = load_index(a.cu_seqlens, b, wide_cu);
+    blocks = a.cu_blocks[b];
+  } else {
+    while (b < a.batch - 1) {
+      const int64_t end = load_index(a.cu_seqlens, b + 1, wide_cu);
+      if (end > r) break;
+      blocks += (end - start + a.block_q - 1) / a.block_q;
+      start = end;
+      ++b;
+    }
+  }
+  const int64_t local = r - start;
+  a.row_req[r] = min(wrap_slot(load_index(a.slot_ids, b, a.wide & kWideSlot), a.max_slots), (int64_t)a.reqs - 1);
+  a.row_seq[r] = min((int32_t)load_index(a.seq_lens, b, a.wide & kWideSeq), a.width);
+  a.row_qpos[r] = (int32_t)(load_index(a.prefix_lens, b, a.wide & kWidePrefix) + local);
+  a.row_idx[r] = (int32_t)min(blocks + local / a.block_q, (int64_t)a.list_rows - 1);
+}
+
 }  // namespace
 }  // namespace xt
 
@@ -683,5 +733,24 @@ extern "C" int xt_minimax_prefill_scores(const void* q, int64_t q_token_stride, 
     XT_PREFILL(16, 2);
   }
 #undef XT_PREFILL
+  return check_launch(what);
+}
+
+extern "C" int xt_block_prefill_rows(const void* cu_seqlens, const void* slot_ids, const void* prefix_lens,
+                                     const void* seq_lens, const int64_t* cu_seqblocks, int index_int64, int batch,
+                                     int rows, int block_q, int64_t max_slots, int reqs, int width, int list_rows,
+                                     int64_t* row_req, int32_t* row_seq, int32_t* row_qpos, int32_t* row_idx,
+                                     xt_stream_t stream) {
+  const char* what = "xt_block_prefill_rows";
+  if (batch < 0 || rows < 0) return fail(XT_EINVAL, "%s: negative size", what);
+  if (batch == 0 || rows == 0) return ok();
+  if (!cu_seqlens || !slot_ids || !prefix_lens || !seq_lens || !row_req || !row_seq || !row_qpos || !row_idx)
+    return fail(XT_EINVAL, "%s: a required pointer is null", what);
+  if (block_q <= 0 || max_slots <= 0 || reqs <= 0 || width < 0 || list_rows <= 0)
+    return fail(XT_EINVAL, "%s: block size, slots, table and list rows must be positive", what);
+  const RowArgs a = {cu_seqlens, slot_ids, prefix_lens, seq_lens, cu_seqblocks, index_int64, batch, rows, block_q,
+                     max_slots, reqs, width, list_rows, row_req, row_seq, row_qpos, row_idx};
+  hipLaunchKernelGGL(prefill_rows_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), a);
   return check_launch(what);
 }

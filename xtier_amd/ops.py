@@ -493,6 +493,37 @@ def _pages(pay, sc, what):
     return pay, sc
 
 
+def _block_prefill_rows(cu_seqlens, slot_ids, prefix_lens, seq_lens, cu_seqblocks, total_q, block_q, max_slots,
+                        req_to_token, list_rows):
+    """(row_req int64, row_seq, row_qpos, row_idx int32), each [total_q]: request row (wrapped as the reference wraps it,
+    then kept inside the table), length within the table, position and list row of each query of a ragged batch, on the
+    device without a synchronization (xt_block_prefill_rows)."""
+    dev = cu_seqlens.device
+    batch = min(cu_seqlens.shape[0] - 1, *(t.shape[0] for t in (slot_ids, prefix_lens, seq_lens, cu_seqblocks)
+                                           if t is not None))
+    if batch <= 0 and total_q:
+        raise ValueError('xtier_amd.fp4_prefill_gqa_share_sparse: queries without a request')
+    wide, index = 0, []
+    for bit, t in ((16, cu_seqlens), (4, slot_ids), (8, prefix_lens), (2, seq_lens)):
+        if t.dtype != torch.int32:
+            t = t if t.dtype == torch.int64 else t.to(torch.int64)
+            wide |= bit
+        index.append(t if t.is_contiguous() else t.contiguous())
+    if cu_seqblocks is not None:
+        cu_seqblocks = cu_seqblocks.to(torch.int64).contiguous()
+    elif batch > 64:   # the kernel's walk over the requests before a row would be longer than these launches
+        cu = index[0].to(torch.int64)
+        nblk = (cu[1:] - cu[:-1] + block_q - 1) // block_q
+        cu_seqblocks = torch.cat([torch.zeros(1, dtype=torch.int64, device=dev), torch.cumsum(nblk, 0)])
+    row_req = torch.empty(total_q, dtype=torch.int64, device=dev)
+    row_seq, row_qpos, row_idx = torch.empty((3, total_q), dtype=torch.int32, device=dev).unbind(0)
+    _lib.check(_lib.lib().xt_block_prefill_rows(
+        *map(_ptr, index), _ptr(cu_seqblocks), wide, batch, total_q, int(block_q), max_slots, req_to_token.shape[0],
+        req_to_token.shape[1], list_rows, _ptr(row_req), _ptr(row_seq), _ptr(row_qpos), _ptr(row_idx),
+        _stream(cu_seqlens)), 'fp4_prefill_gqa_share_sparse')
+    return row_req, row_seq, row_qpos, row_idx
+
+
 def fp4_prefill_gqa_share_sparse(q, k_cache, v_cache, sink, req_to_token, slot_ids, topk_idx, block_size_q,
                                  block_size_k, cu_seqlens, seq_lens, prefix_lens, max_seqlen_q, sm_scale=None,
                                  use_tma=True, cu_seqblocks_q=None, max_seqblock_q=None, q_scale=None, k_scale=None,
@@ -518,20 +549,9 @@ def fp4_prefill_gqa_share_sparse(q, k_cache, v_cache, sink, req_to_token, slot_i
     _need_cuda(q, k_pay, v_pay, req_to_token, slot_ids, topk_idx, cu_seqlens, seq_lens, prefix_lens, out)
     sm_scale = (d ** -0.5 if sm_scale is None else sm_scale) * (1.0 if q_scale is None else q_scale)
     dev = q.device
-    cu = cu_seqlens.to(torch.int64)
-    if cu_seqblocks_q is None:
-        nblk = (cu[1:] - cu[:-1] + block_size_q - 1) // block_size_q
-        cu_seqblocks_q = torch.cat([torch.zeros(1, dtype=torch.int64, device=dev), torch.cumsum(nblk, 0)])
-    r = torch.arange(total_q, device=dev, dtype=torch.int64)
-    bi = torch.searchsorted(cu[1:].contiguous(), r, right=True)
-    local = r - cu[bi]
-    max_slots = k_pay.shape[0] * block_size_k
-    # wrapped as the reference wraps it, then kept inside the table (on the device: no synchronization)
-    row_req = torch.clamp(torch.remainder(slot_ids.to(torch.int64)[bi], max_slots), max=req_to_token.shape[0] - 1)
-    row_qpos = (prefix_lens.to(torch.int64)[bi] + local).to(torch.int32)
-    row_seq = torch.clamp(seq_lens.to(torch.int32)[bi], max=req_to_token.shape[1])   # positions within the table
-    row_idx = torch.clamp(cu_seqblocks_q.to(torch.int64)[bi] + local // block_size_q,
-                          max=topk_idx.shape[1] - 1).to(torch.int32)   # a list row of topk_idx
+    rows = _block_prefill_rows(cu_seqlens, slot_ids, prefix_lens, seq_lens, cu_seqblocks_q, total_q, block_size_q,
+                               k_pay.shape[0] * block_size_k, req_to_token, topk_idx.shape[1])
+    row_req, row_seq, row_qpos, row_idx = rows
     if q.stride(-1) != 1:
         q = q.contiguous()
     if out is None:
