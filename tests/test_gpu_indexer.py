@@ -49,7 +49,7 @@ def test_topk_rows_values_placed_by_position(cols, k):
     assert np.array_equal(got, ref.topk_rows(x.numpy(), k))
 
 
-@pytest.mark.parametrize('cols', [4095, 4096, 4097, 8192, 8196, 16384, 16385, 32768, 32772, 49152, 49153, 65536, 65540,
+@pytest.mark.parametrize('cols', [1024, 2048, 2049, 4095, 4096, 4097, 8192, 8196, 16384, 16385, 32768, 32772, 49152, 49153, 65536, 65540,
                                   98304, 98305])
 def test_topk_rows_edges_of_the_register_forms(cols):
     """Rows that just fill a form and that are just past it; random, with ties at the threshold, and masked."""
@@ -81,6 +81,19 @@ def test_topk_rows_packed_forms(rows, cols):
         got = ops.topk_rows(x.cuda(), k).cpu().numpy()
         for r in {0, 1, *range(n), rows - 1}:
             assert np.array_equal(got[r:r + 1], ref.topk_rows(x[r:r + 1].numpy(), k)), r
+
+
+@pytest.mark.parametrize('rows,cols,skip', [(3, 4093, 0), (5, 5000, 1), (3, 32767, 3), (2, 65537, 2), (300, 30001, 0),
+                                            (2, 131075, 1)])
+def test_topk_rows_off_16_byte_alignment(rows, cols, skip):
+    """Rows whose stride or base is not a multiple of 16 bytes."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn(rows * cols + skip, generator=g)
+    x[skip + 1::97] = -math.inf
+    got = ops.topk_rows(x.cuda()[skip:].view(rows, cols), 2048).cpu().numpy()
+    n = min(rows, 5)
+    assert np.array_equal(got[:n], ref.topk_rows(x[skip:].view(rows, cols)[:n].numpy(), 2048))
+    assert np.array_equal(got[-1:], ref.topk_rows(x[skip:].view(rows, cols)[-1:].numpy(), 2048))
 
 
 def test_topk_rows_empty_rows():

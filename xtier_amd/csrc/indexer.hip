@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* x,
   for (int i = (int)k + tid; i < topk; i += kTopkThreads) o[i] = -1;
 }
 
-// Rows of at most kTopkRegMax columns (16-byte aligned rows): the row is read once into registers as order keys (a
+// Rows of at most kTopkRegMax columns: the row is read once into registers as order keys (a
 // non-finite value as key 0, which no finite value has; the smallest finite key is 0x00800000). Chunk i of thread t
 // holds columns 4 (TH i + t) .. + 3.
 //   1. A histogram of the top 13 bits finds the bucket b0 that holds the topk-th largest key (counted as the row
@@ -175,6 +175,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* x,
 // row fills it or not, so a row takes the smallest form that holds it (xt_topk_rows). Measured per call at 512 keys,
 // the form of 98304 columns -> the smallest: 4096 columns 26.7 us -> 8.3 us (1 row), 54.4 us -> 10.0 us (352 rows,
 // several workgroups to a CU); 32768 columns 26.4 us -> 15.4 us (32 rows).
+// a 16-byte load of dword alignment, all that these loads need: rows of any stride take the register forms (32 rows x
+// 32767 columns 59.6 us -> 15.4 us, 352 x 95087 254 us -> 46 us, against streaming them)
+typedef float4_t float4_dw_t __attribute__((aligned(4)));
 constexpr int kTopkRegMax = 4 * 1024 * 48;   // columns of the largest form
 
 template <int NW>
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
   const auto load = [&](int i, uint32_t (&v4)[4]) {   // chunk i of the row, as bits
     const int c = 4 * (TH * i + tid);
     if (ALIGNED4 || 4 * TH * (i + 1) <= cols) {   // uniform: the whole chunk row is inside the row, or clamped into it
-      const float4_t v = *reinterpret_cast<const float4_t*>(xr + (ALIGNED4 ? min(c, cols - 4) : c));
+      const float4_dw_t v = *reinterpret_cast<const float4_dw_t*>(xr + (ALIGNED4 ? min(c, cols - 4) : c));
       v4[0] = __float_as_uint(v[0]); v4[1] = __float_as_uint(v[1]);
       v4[2] = __float_as_uint(v[2]); v4[3] = __float_as_uint(v[3]);
     } else {   // an address inside the row; columns past the end are masked when converted
@@ -1107,10 +1110,11 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
   if (rows == 0 || topk == 0) return ok();
   if (!out || (!x && cols > 0)) return fail(XT_EINVAL, "%s: a required pointer is null", what);
   if (ld < cols || out_ld < topk) return fail(XT_EINVAL, "%s: row strides shorter than the rows", what);
-  // the register-resident rows read at column 0 (and at cols - 4 when cols % 4 == 0); empty rows stream, reading
-  // nothing, and come out all -1
+  // empty rows stream, reading nothing, and come out all -1
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (cols > 0 && cols <= kTopkRegMax && ld % 4 == 0 && aligned(x, 16)) {
+  // short rows stream: the 8192-bucket histogram costs more than the passes it saves (601 columns: 6.3 us against 9.2 us;
+  // 4093: 11.6 us against 8.8 us at 32 rows, 17.2 us against 10.1 us at 352)
+  if (cols > (rows > device_cus() ? 1024 : 2048) && cols <= kTopkRegMax) {
     const auto go = [&](auto kernel, int threads) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3((unsigned)threads), 0, st, x, ld, cols, topk, out, out_ld);
     };
