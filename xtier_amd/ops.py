@@ -546,7 +546,8 @@ def fp4_prefill_gqa_share_sparse(q, k_cache, v_cache, sink, req_to_token, slot_i
     if k_pay.shape[3] * 2 != d or qh % kh:
         raise ValueError(f'xtier_amd.fp4_prefill_gqa_share_sparse: q {tuple(q.shape)} does not fit pages '
                          f'{tuple(k_pay.shape)}')
-    _need_cuda(q, k_pay, v_pay, req_to_token, slot_ids, topk_idx, cu_seqlens, seq_lens, prefix_lens, out)
+    _need_cuda(q, k_pay, v_pay, k_sc8, v_sc8, req_to_token, slot_ids, topk_idx, cu_seqlens, seq_lens, prefix_lens,
+               cu_seqblocks_q, out)
     sm_scale = (d ** -0.5 if sm_scale is None else sm_scale) * (1.0 if q_scale is None else q_scale)
     dev = q.device
     rows = _block_prefill_rows(cu_seqlens, slot_ids, prefix_lens, seq_lens, cu_seqblocks_q, total_q, block_size_q,
