@@ -395,11 +395,12 @@ int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int topk, int32
                  xt_stream_t stream);
 
 /* The per-row arguments of xt_block_sparse_prefill_nvfp4 for a ragged batch (kv_fp4.py:384-400): row r belongs to the
- * request b whose rows are cu_seqlens[b] .. cu_seqlens[b + 1] - 1 (the last request takes rows past the end). row_req =
- * slot_ids[b] wrapped into max_slots, at most reqs - 1; row_seq = seq_lens[b], at most width; row_qpos = prefix_lens[b]
- * + the row's offset; row_idx = cu_seqblocks[b] + offset / block_q, at most list_rows - 1. cu_seqblocks [batch + 1] may
- * be NULL: the requests' rows in whole blocks of block_q. index_int64: bit 1 seq_lens, 2 slot_ids, 3 prefix_lens, 4
- * cu_seqlens are int64 (else int32). */
+ * request b whose rows are cu_seqlens[b] .. cu_seqlens[b + 1] - 1. row_req = slot_ids[b] wrapped into max_slots, at most
+ * reqs - 1; row_seq = seq_lens[b], at most width; row_qpos = prefix_lens[b] + the row's offset; row_idx =
+ * cu_seqblocks[b] + offset / block_q, at most list_rows - 1. A row at or past cu_seqlens[batch] has no request: its
+ * row_seq is 0, so it has no keys. cu_seqblocks [batch] may be NULL: the requests' rows in whole blocks of block_q.
+ * index_int64: bit 1 seq_lens, 2 slot_ids, 3 prefix_lens, 4 cu_seqlens are int64 (else int32); bit 5: cu_seqlens is
+ * [batch], the last request takes every row from its start on. */
 int xt_block_prefill_rows(const void* cu_seqlens, const void* slot_ids, const void* prefix_lens, const void* seq_lens,
                           const int64_t* cu_seqblocks, int index_int64, int batch, int rows, int block_q,
                           int64_t max_slots, int reqs, int width, int list_rows, int64_t* row_req, int32_t* row_seq,

@@ -8,11 +8,15 @@ from xtier_amd import ops
 PAGES, KH, BLOCK, D = 4, 2, 128, 128
 
 
+class Reached(Exception):
+    """A library entry was about to be called."""
+
+
 @pytest.fixture(autouse=True)
 def no_launch(monkeypatch):
     class Library:
         def __getattr__(self, name):
-            pytest.fail(f'{name} was reached')
+            raise Reached(name)
     monkeypatch.setattr(ops._lib, 'lib', Library)
 
 
@@ -42,4 +46,25 @@ def test_each_tensor_must_be_on_the_gpu(monkeypatch, name):
             raise ValueError('on the host')
     monkeypatch.setattr(ops, '_need_cuda', need_cuda)
     with pytest.raises(ValueError, match='on the host'):
+        ops.fp4_prefill_gqa_share_sparse(**kw)
+
+
+@pytest.mark.parametrize('cu,n,blocks', [([0, 3, 5], 1, None), ([0, 3, 5], 0, None), ([0, 0, 5], 1, [0, 0, 5]),
+                                         ([0, 3, 5], 2, [0]), ([0, 2, 4, 5], 2, [0, 2, 4, 5])])
+def test_arrays_short_of_the_requests_with_rows_are_refused(monkeypatch, cu, n, blocks):
+    """They were indexed out of bounds once; taken as they are, another request's keys would answer."""
+    monkeypatch.setattr(ops, '_need_cuda', lambda *tensors: None)
+    with pytest.raises(ValueError, match='requests'):
+        ops.fp4_prefill_gqa_share_sparse(**_args(cu, n, blocks))
+
+
+@pytest.mark.parametrize('cu,n,blocks', [([0, 3, 5], 2, None), ([0, 3, 5, 5, 5], 2, None), ([0, 3, 5, 5], 2, [0, 3, 5]),
+                                         ([0, 3, 5], 4, None), ([0], 1, None)])
+def test_arrays_that_cover_every_row_are_taken(monkeypatch, cu, n, blocks):
+    """Requests without rows at the end need no entries, and longer arrays do no harm."""
+    monkeypatch.setattr(ops, '_need_cuda', lambda *tensors: None)
+    kw = _args(cu, n, blocks)
+    if not kw['q'].shape[0]:
+        kw['q'] = torch.zeros(2, 2 * KH, D, dtype=torch.bfloat16)
+    with pytest.raises(Reached, match='xt_block_prefill_rows'):
         ops.fp4_prefill_gqa_share_sparse(**kw)

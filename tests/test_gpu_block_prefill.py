@@ -112,6 +112,33 @@ def test_row_arguments(batch, bq, given, wide):
         assert torch.equal(x.cpu().long(), y)
 
 
+@pytest.mark.parametrize('batch', [3, 70])
+@pytest.mark.parametrize('extra,given', [(0, True), (0, False), (1, True), (1, False), (5, False), (-2, False)])
+def test_row_arguments_of_rows_past_the_last_end(batch, extra, given):
+    """Rows at or past cu_seqlens[-1]: of the next request where the arrays hold one (`extra` entries beyond the ends),
+    else without keys. With fewer entries than ends the last requests have no rows. The walk and the search."""
+    g = torch.Generator().manual_seed(batch + extra)
+    n = torch.randint(1, 40, (batch,), generator=g)
+    if extra < 0:
+        n[extra:] = 0
+    cu = torch.cat([torch.zeros(1, dtype=torch.int64), n.cumsum(0)])
+    past, total, entries, bq = int(cu[-1]), int(cu[-1]) + (0 if extra < 0 else 300), batch + extra, 7
+    sid = torch.randint(-256, 256, (entries,), generator=g)
+    pre, seq = torch.randint(0, 5000, (entries,), generator=g), torch.randint(1, 9000, (entries,), generator=g)
+    blk = torch.cat([torch.zeros(1, dtype=torch.int64), ((n + bq - 1) // bq).cumsum(0)])
+    r2t = torch.empty(100, 6000, dtype=torch.int32)
+    got = [x.cpu().long() for x in
+           ops._block_prefill_rows(cu.int().cuda(), sid.cuda(), pre.int().cuda(), seq.int().cuda(),
+                                   blk.int().cuda() if given else None, total, bq, 256, r2t, 1 << 20)]
+    r = torch.arange(total if extra > 0 else past)
+    b = torch.searchsorted(cu[1:].contiguous(), r, right=True)
+    local = r - cu[b]
+    for x, y in zip(got, ((sid[b] % 256).clamp(max=99), seq[b].clamp(max=6000), pre[b] + local, blk[b] + local // bq)):
+        assert torch.equal(x[:len(r)], y)
+    for x, y in zip(got, (0, 0, -1, 0)):
+        assert (x[len(r):] == y).all()
+
+
 def test_strided_pool_kv_scale_and_queries_without_keys():
     print('block-sparse prefill: strided pool, kv_scale, empty rows', flush=True)
     c = _case(77, q_lens=(40, 70), prefix=(300, 129), bq=16, topk=3)

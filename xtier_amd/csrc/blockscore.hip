@@ -32,7 +32,7 @@ constexpr int kPoolRows = 128;   // slots per page of the index pool
 constexpr int kScoreWaves = 4;
 
 // index arrays given as int32 or int64 (bit i of `wide` set: argument i is int64)
-enum : int { kWideR2t = 1, kWideSeq = 2, kWideSlot = 4, kWidePrefix = 8, kWideCu = 16 };
+enum : int { kWideR2t = 1, kWideSeq = 2, kWideSlot = 4, kWidePrefix = 8, kWideCu = 16, kOpenEnd = 32 };
 
 __device__ inline int64_t load_index(const void* p, int64_t i, bool wide) {
   return wide ? static_cast<const int64_t*>(p)[i] : (int64_t) static_cast<const int32_t*>(p)[i];
@@ -500,11 +500,12 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The per-row arguments of a ragged block-sparse prefill (kv_fp4.py:384-400 derives them per program): thread = row.
+// The per-row arguments of a ragged block-sparse prefill (kv_fp4.py:384-400 derives them per program): thread = row. A
+// row at or past cu_seqlens[batch] is no request's and gets no keys, unless the last request's end is open.
 
 struct RowArgs {
-  const void *cu_seqlens, *slot_ids, *prefix_lens, *seq_lens;   // [batch + 1], [batch] ...
-  const int64_t* cu_blocks;   // [batch + 1] query blocks before each request, or NULL: from cu_seqlens
+  const void *cu_seqlens, *slot_ids, *prefix_lens, *seq_lens;   // [batch + 1] ([batch], open end), [batch] ...
+  const int64_t* cu_blocks;   // [batch] query blocks before each request, or NULL: from cu_seqlens
   int wide;
   int batch, rows, block_q;
   int64_t max_slots;
@@ -517,11 +518,13 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const RowArgs a) {
   const int r = (int)blockIdx.x * 256 + (int)threadIdx.x;
   if (r >= a.rows) return;
   const bool wide_cu = a.wide & kWideCu;
-  // the request: how many of cu[1:] are at or below r; without cu_blocks the walk counts the blocks on its way
+  // the request: how many of the ends cu[1 .. ends] are at or below r; without cu_blocks the walk counts the blocks on
+  // its way
+  const int ends = a.batch - (a.wide & kOpenEnd ? 1 : 0);
   int b = 0;
   int64_t start = load_index(a.cu_seqlens, 0, wide_cu), blocks = 0;
   if (a.cu_blocks) {
-    int n = a.batch - 1;   // of cu[1 .. batch - 1]: the last request takes every row left
+    int n = ends;
     while (n > 0) {
       const int half = n / 2;
       if (load_index(a.cu_seqlens, b + half + 1, wide_cu) <= r) {
@@ -531,16 +534,24 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const RowArgs a) {
         n = half;
       }
     }
-    start = load_index(a.cu_seqlens, b, wide_cu);
-    blocks = a.cu_blocks[b];
+    if (b < a.batch) {
+      start = load_index(a.cu_seqlens, b, wide_cu);
+      blocks = a.cu_blocks[b];
+    }
   } else {
-    while (b < a.batch - 1) {
+    while (b < ends) {
       const int64_t end = load_index(a.cu_seqlens, b + 1, wide_cu);
       if (end > r) break;
       blocks += (end - start + a.block_q - 1) / a.block_q;
       start = end;
       ++b;
     }
+  }
+  if (b >= a.batch) {
+    a.row_req[r] = 0;
+    a.row_seq[r] = a.row_idx[r] = 0;
+    a.row_qpos[r] = -1;
+    return;
   }
   const int64_t local = r - start;
   a.row_req[r] = min(wrap_slot(load_index(a.slot_ids, b, a.wide & kWideSlot), a.max_slots), (int64_t)a.reqs - 1);

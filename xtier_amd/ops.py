@@ -497,13 +497,19 @@ def _block_prefill_rows(cu_seqlens, slot_ids, prefix_lens, seq_lens, cu_seqblock
                         req_to_token, list_rows):
     """(row_req int64, row_seq, row_qpos, row_idx int32), each [total_q]: request row (wrapped as the reference wraps it,
     then kept inside the table), length within the table, position and list row of each query of a ragged batch, on the
-    device without a synchronization (xt_block_prefill_rows)."""
+    device without a synchronization (xt_block_prefill_rows). Arrays with an entry more than cu_seqlens has ends give
+    the rows from cu_seqlens[-1] on to that request; otherwise those rows have no keys. Arrays too short for the
+    requests that have rows are refused, which takes a synchronization (inside a graph capture, where none is possible,
+    such rows have no keys)."""
     dev = cu_seqlens.device
-    batch = min(cu_seqlens.shape[0] - 1, *(t.shape[0] for t in (slot_ids, prefix_lens, seq_lens, cu_seqblocks)
-                                           if t is not None))
-    if batch <= 0 and total_q:
-        raise ValueError('xtier_amd.fp4_prefill_gqa_share_sparse: queries without a request')
-    wide, index = 0, []
+    ends = cu_seqlens.shape[0] - 1
+    entries = min(t.shape[0] for t in (slot_ids, prefix_lens, seq_lens, cu_seqblocks) if t is not None)
+    batch = min(entries, ends + 1)
+    short = entries < ends and not (dev.type == 'cuda' and torch.cuda.is_current_stream_capturing())
+    if total_q and (batch <= 0 or (short and int(cu_seqlens[entries]) < total_q)):
+        raise ValueError(f'xtier_amd.fp4_prefill_gqa_share_sparse: slot_ids, prefix_lens, seq_lens or cu_seqblocks_q '
+                         f'hold {entries} requests, the queries are of more')
+    wide, index = 32 if batch > ends else 0, []   # 32: an open end
     for bit, t in ((16, cu_seqlens), (4, slot_ids), (8, prefix_lens), (2, seq_lens)):
         if t.dtype != torch.int32:
             t = t if t.dtype == torch.int64 else t.to(torch.int64)
