@@ -704,12 +704,23 @@ def _mla_keys(indices, lengths, rows):
 def default_mla_splits(rows, topk, v4=False):
     """Key splits per row for sparse MLA: as many as keep every workgroup in one round on the CUs (a CU holds one
     workgroup, so one more would double the time: 96 rows, top-1024, 128 heads 78 us with 3 splits, 56.5 us with 2; 200
-    rows, top-640, 95 us with 2, 57 us with 1), with at least 128 keys per split up to 8 splits and 256 beyond, none for
-    lists of up to 256 keys (the merge costs more: 61 rows 27.9 us with 2 splits, 21.3 us with 1), and at least enough
-    that a split's slot list fits in LDS beside the key and query tiles. Measured on MI355X (256 CUs), 64 heads: 61 rows,
-    top-640 34.3 us with 2 splits, 30.0 us with 4; 16 rows, top-512 25.1 us with 2, 20.7 us with 4."""
+    rows, top-640, 95 us with 2, 57 us with 1), with at least 128 keys per split up to 8 splits and 256 beyond, and at
+    least enough that a split's slot list fits in LDS beside the key and query tiles. Measured on MI355X (256 CUs), 64
+    heads: 61 rows, top-640 34.3 us with 2 splits, 30.0 us with 4; 16 rows, top-512 25.1 us with 2, 20.7 us with 4.
+
+    Lists of fewer than 512 keys keep one split. On the NVFP4 latent the FP32 accumulators then go straight to the
+    output; a split's partial is FP16 (61 rows, top-384: FP16 output 2.3e-4 from 64 bits with 1 split, 2.8e-4 with 3;
+    top-512 2.8e-4 with 2 splits, 2.7e-4 with 4). The pages' partials are FP32, but from 33 rows on the merge costs what
+    the split gains (64 rows, top-320, 64 heads 25.2 us with 1, 30.0 us with 2; 85 rows, top-384, 128 heads 36.7 us with
+    1, 41.6 us with 3), so they split from 384 keys with at most a row for every 8 CUs (24 rows, top-384 26.7 us with 1,
+    23.2 us with 3; 32 rows, top-511, 128 heads 43.6 us with 1, 36.8 us with 3).
+
+    The number of splits moves the result within its rounding: each split rounds its probabilities (BF16 for the pages,
+    FP16 for the latent) against its own running maximum. Pages, 61 rows of 640 keys: 2.15e-3 from 64 bits with 2
+    splits, 2.10e-3 with 4, and 2e-3 between the two; 200 rows: 2.15e-3 with 2, 2.19e-3 with 1."""
     fit = math.ceil(topk / _lib.lib().xt_sparse_mla_max_split_keys(int(v4)))
-    most = 1 if topk <= 256 else max(min(8, topk // 128), topk // 256)
+    least = 384 if v4 and 8 * rows <= device_cus() else 512
+    most = 1 if topk < least else max(min(8, topk // 128), topk // 256)
     return min(64, max(1, min(device_cus() // max(1, rows), most), fit))
 
 
