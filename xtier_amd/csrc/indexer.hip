@@ -698,9 +698,11 @@ __global__ __launch_bounds__(64 * kQsaWaves, 2) void qsa_logits_lds_kernel(const
       qb[g][kk] = __builtin_bit_cast(short8_t, *reinterpret_cast<const xt_u32x4_t*>(qp + 16 * kk));
   }
   // Logit (g, o) of a lane is that of row rw + g kRowsG + first(o) + h half: for H <= 4 a row's heads are H consecutive
-  // C elements of one lane, for H >= 8 the halves split pairs of rows.
-  constexpr int half = H <= 4 ? 4 / H : 1;
-  const auto first = [](int o) { return H <= 4 ? (8 * (o * H >> 2) + (o * H & 3)) / H : 2 * o; };
+  // C elements of one lane, for H >= 8 the halves split pairs of rows (32 heads: one row, which the lower half stores).
+  constexpr int half = H <= 4 ? 4 / H : H == 32 ? 0 : 1;
+  const auto first = [](int o) constexpr { return H <= 4 ? (8 * (o * H >> 2) + (o * H & 3)) / H : 2 * o; };
+  static_assert((kQsaWaves - 1) * kRowsW + (G - 1) * kRowsG + first(kOut - 1) + half < kRowsWg,
+                "the last lane's last row is one of the workgroup's (an entry of range)");
   int max_start = 0, min_end = 0x7FFFFFFF, lo = 0x7FFFFFFF, hi = 0;
   for (int r = rw + lane; r < min(rw + kRowsW, a.rows); r += 64) {
     const int st = a.starts[r], en = a.ends[r];
