@@ -171,6 +171,30 @@ def test_prefill_scores_many_row_tiles(prefix, ext, dim, bs, heads, q_dtype):
     test_prefill_scores(prefix, ext, dim, bs, heads, q_dtype)
 
 
+@pytest.mark.parametrize('factor', [-1.0, 0.0])
+def test_prefill_scores_with_a_factor_that_is_not_positive(factor):
+    """The maximum is of the scaled values, so a negative factor takes the smallest product."""
+    dim, bs, heads, ext, pre = 128, 128, 4, 200, 700
+    g = torch.Generator().manual_seed(7)
+    r2t, pages = _mapping([ext + pre], g)
+    pay, sc = _pool(pages, dim, g)
+    q = (torch.randn(ext, heads, dim, generator=g) * 0.3).to(torch.bfloat16)
+    one = lambda *v: torch.tensor(v, dtype=torch.int32)  # noqa: E731
+    score = torch.full((heads, ext, -(-(ext + pre) // bs)), 7.0, device='cuda')
+    ops.minimax_prefill_scores(q.cuda(), pay.cuda(), sc.cuda(), r2t.cuda(), score, one(0, ext).cuda(),
+                               one(ext + pre).cuda(), one(pre).cuda(), one(0).cuda(), bs, factor * dim ** -0.5, 1.0, ext)
+    got = score.cpu().numpy().astype(np.float64)
+    want = ref.minimax_block_scores_prefill(q.float().numpy(), pay.numpy(), sc.numpy(), r2t.numpy(), [0], [0, ext],
+                                            [ext + pre], [pre], bs, factor * dim ** -0.5, 1.0)
+    assert np.array_equal(np.isnan(want), got == 7.0) and np.array_equal(np.isneginf(want), np.isneginf(got))
+    c, keys = abs(ops.minimax_score_factor(factor * dim ** -0.5, 1.0)), np.abs(_keys(pay, sc))
+    for t in range(ext):
+        bound = _block_bound(q[t].float().numpy(), keys, r2t[0].long().numpy(), ext + pre, bs, c)
+        f = np.isfinite(want[:, t])
+        err = np.abs(got[:, t][f] - want[:, t][f])
+        assert (err <= (bound + 2.0 ** -23 * np.abs(want[:, t]))[f]).all(), t
+
+
 @pytest.mark.parametrize('dim,heads,bs,score_type,q_dtype', [
     (128, 1, 32, 'max', torch.bfloat16), (128, 3, 64, 'lse', torch.float16), (128, 4, 256, 'max', torch.float16),
     (128, 5, 128, 'max', torch.bfloat16), (64, 8, 128, 'lse', torch.bfloat16), (64, 7, 256, 'max', torch.bfloat16),

@@ -484,10 +484,10 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
         }
       }
     }
-    if (++sub == subs) {   // the block is complete: max(round(c x)) = round(c max(x)) for c > 0
+    if (++sub == subs) {   // the block is complete: max(round(c x)) = round(c max(x)) for c > 0 (else mr is -inf, unused)
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const float v = swap32_max(fmaxf(m[g], mr[g] * a.c));
+        const float v = swap32_max(a.c > 0.0f ? fmaxf(m[g], mr[g] * a.c) : m[g]);
         const int64_t row = row0 + RG * (G * wave + g) + j / HPW;
         if (h == 0 && bi < nblk[g])
           store_score(a, (int64_t)head * a.s_hs + (q0 + row) * a.s_ns + (blk_lo + bi) * a.s_ks, v);
