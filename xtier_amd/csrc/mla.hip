@@ -295,8 +295,8 @@ __device__ inline int64_t part_index(const MlaArgs& a, int64_t row, int split, i
   return ((((row * a.splits + split) * waves + wave) * 16 + k) * 64 + lane) * 8;
 }
 
-// TL: the per-wave timeline build (xt_mla_timeline), launched only while a stamp buffer is set, so the kernel the
-// serving path runs carries none of its instructions or registers.
+// TL: the per-wave timeline build (xt_mla_timeline) of each form, launched only while a stamp buffer is set, so the kernel
+// the serving path runs carries none of its instructions or registers.
 // PART: launches with whole waves of absent heads (heads <= 112) or with list lengths: a wave without a live head only
 // dequantizes, so the others have the matrix cores and the LDS to themselves, and a step without a valid key is
 // dequantized only. 64 heads: 1024 rows of 2048 keys (NVFP4) 576 us -> 431 us, 61 rows of 640 keys (V4, lists three
@@ -738,6 +738,15 @@ size_t mla_workspace_bytes(int rows, int heads, int splits, size_t part_elem) {
 std::atomic<uint64_t*> g_mla_timeline{nullptr};
 std::atomic<size_t> g_mla_timeline_bytes{0};
 
+template <int F>
+void (*mla_form(bool two, bool timeline, bool part))(const MlaArgs) {
+  if (timeline)
+    return two ? (part ? mla_kernel<F, true, true, true> : mla_kernel<F, true, true, false>)
+               : (part ? mla_kernel<F, false, true, true> : mla_kernel<F, false, true, false>);
+  return two ? (part ? mla_kernel<F, true, false, true> : mla_kernel<F, true, false, false>)
+             : (part ? mla_kernel<F, false, false, true> : mla_kernel<F, false, false, false>);
+}
+
 // Everything but the caches: checks, key lists, split sizing, workspace carving and the launches.
 template <int F>
 int mla_launch(const char* what, MlaArgs& a, bool extra, const void* q, int64_t q_row_stride, int64_t q_head_stride,
@@ -794,12 +803,8 @@ int mla_launch(const char* what, MlaArgs& a, bool extra, const void* q, int64_t 
                             : 0u;
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)n_units), block(64 * kMWaves);
-  const bool tl = a.stamps != nullptr;
-  const bool part = !tl && (heads <= kMHeads - 16 || a.len[0] || a.len[1]);
-  void (*const fn)(const MlaArgs) = extra ? (tl ? mla_kernel<F, true, true, false> : part ? mla_kernel<F, true, false, true>
-                                                                                   : mla_kernel<F, true, false, false>)
-                                          : (tl ? mla_kernel<F, false, true, false> : part ? mla_kernel<F, false, false, true>
-                                                                                    : mla_kernel<F, false, false, false>);
+  const bool part = heads <= kMHeads - 16 || a.len[0] || a.len[1];
+  void (*const fn)(const MlaArgs) = mla_form<F>(extra, a.stamps != nullptr, part);
   if (int e = allow_lds(reinterpret_cast<const void*>(fn), lds_bytes, what)) return e;
   hipLaunchKernelGGL(fn, grid, block, lds_bytes, st, a);
   if (splits > 1) {
