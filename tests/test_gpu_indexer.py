@@ -298,6 +298,47 @@ def test_dsa_paged_logits_edges(heads, dim, block, msl):
             assert (got[r, n:] == fill).all(), r
 
 
+@pytest.mark.parametrize('rows,heads,dim,block,msl,run', [
+    (32, 32, 128, 64, 4096, 2), (48, 64, 128, 32, 4096, 3), (41, 32, 256, 96, 5000, 4), (24, 128, 64, 64, 6001, 3),
+    (80, 96, 64, 128, 4095, 5), (64, 32, 128, 64, 65536, 64), (65, 64, 64, 256, 65536 + 33, 64)])
+def test_dsa_paged_logits_runs_of_blocks(rows, heads, dim, block, msl, run):
+    """Runs of several 32-key blocks per wavefront, up to the 64 table entries it holds: lengths that end at every block
+    of a run and inside it, pages crossed within a run, bad table entries in its middle. Every key against FP64."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert min(64, -(-(-(-msl // 32) * rows) // (8 * cus))) == run or cus != 256   # as the launch sizes it
+    g = torch.Generator().manual_seed(rows + heads + msl)
+    width, pages = -(-msl // block), 37
+    vals, scl = _fp8((pages, block, dim), g), torch.rand(pages, block, generator=g) + 0.5
+    kv = torch.empty(pages, block * (dim + 4), dtype=torch.uint8)
+    kv[:, :block * dim] = vals.view(torch.uint8).reshape(pages, -1)
+    kv[:, block * dim:] = scl.view(torch.uint8).reshape(pages, -1)
+    table = torch.randint(0, pages, (rows, width), generator=g, dtype=torch.int32)
+    bad = torch.rand(rows, width, generator=g)
+    table[bad < 0.03], table[bad > 0.97] = -1, pages
+    table[-1, width // 2] = 2 ** 31 - 1
+    r = torch.arange(rows)
+    lens = (msl // 2 // (32 * run) * run + r % (run + 1)) * 32 + torch.tensor([0, 1, 17, 31])[r // (run + 1) % 4]
+    lens[::5] = msl
+    lens[1], lens[2], lens[3] = 0, 32 * run + 1, msl + 500
+    q, w = _fp8((rows, 1, heads, dim), g), torch.randn(rows, heads, generator=g)
+    qd, kd = q[:, 0].cuda().double(), vals.view(-1, dim).cuda().double()
+    wd, sd = w.cuda().double(), scl.view(-1).cuda().double()
+    n = lens.clamp(max=min(msl, width * block)).cuda().view(-1, 1)
+    at = torch.arange(msl, device='cuda')
+    page = table.cuda().long().clamp(min=0)[:, (at // block).clamp(max=width - 1)]
+    live = (at < n) & (page < pages)
+    slot = page.clamp(max=pages - 1) * block + at % block
+    for clean in (False, True):
+        got = ops.dsa_paged_mqa_logits(q.cuda(), kv.view(pages, block, 1, dim + 4).cuda(), w.cuda(), lens.int().cuda(),
+                                       table.cuda(), None, msl, clean).double()
+        for i in range(rows):
+            score = (torch.clamp(qd[i] @ kd.T, min=0) * wd[i].view(-1, 1)).sum(0) * sd
+            bound = ((qd[i].abs() @ kd.abs().T) * wd[i].abs().view(-1, 1)).sum(0) * sd * ((dim + heads + 4) * 2.0 ** -24)
+            ok = live[i]
+            assert (got[i][ok] - score[slot[i][ok]]).abs().le(bound[slot[i][ok]] + 1e-30).all(), i
+            assert (got[i][~ok] == (-math.inf if clean else 0.0)).all(), i
+
+
 def test_glm_schedule_and_sm_count():
     assert glm.get_paged_mqa_logits_metadata(None, 1, 2, x=3) is None
     assert glm.get_num_sms(None) == torch.cuda.get_device_properties(0).multi_processor_count
