@@ -151,6 +151,59 @@ def test_qsa_indexer_logits_edges_of_the_tiles(rows, heads, dim, keys, dtype):
     test_qsa_indexer_logits(rows, heads, dim, keys, dtype)
 
 
+def _check_qsa(logits, q, k, starts, ends, scale):
+    """Every logit against FP64 on the GPU, within the FP32 summation bound (_bound_qsa)."""
+    heads, dim, keys = q.shape[1], q.shape[2], k.shape[0]
+    kd, at = k.double(), torch.arange(keys, device='cuda')
+    for r in range(q.shape[0]):
+        qd = q[r].double()
+        want = torch.clamp(qd @ kd.T, min=0).sum(0) / scale
+        bound = (qd.abs().sum(0) @ kd.abs().T) * ((dim + heads + 2) * 2.0 ** -24 / scale) + want * 2.0 ** -23
+        ok = (at >= int(starts[r])) & (at < int(ends[r]))
+        assert (logits[r].double()[ok] - want[ok]).abs().le(bound[ok]).all(), r
+        assert (logits[r][~ok] == -math.inf).all(), r
+
+
+def _qsa_case(rows, heads, dim, keys, dtype):
+    g = torch.Generator().manual_seed(rows * keys + heads)
+    q = torch.randn(rows, heads, dim, generator=g).to(dtype).cuda()
+    k = torch.randn(keys, dim, generator=g).to(dtype).cuda()
+    ends = (torch.arange(rows) * (keys // rows) + keys // 3).clamp(max=keys).int()
+    starts = torch.zeros(rows, dtype=torch.int32)
+    starts[rows // 2], ends[0] = keys // 5, keys + 9
+    return q, k, starts, ends
+
+
+@pytest.mark.parametrize('rows,heads,dim,keys,dtype', [
+    (300, 2, 128, 33000, torch.bfloat16), (70, 8, 128, 33001, torch.bfloat16), (70, 8, 64, 40000, torch.float16),
+    (70, 16, 128, 40003, torch.bfloat16), (40, 16, 64, 33000, torch.float16), (30, 32, 64, 50001, torch.bfloat16),
+    (30, 32, 128, 33000, torch.float16), (70, 32, 256, 20001, torch.bfloat16), (130, 8, 256, 20000, torch.bfloat16)])
+def test_qsa_indexer_logits_most_column_groups(rows, heads, dim, keys, dtype):
+    """Enough rows and keys for four column groups per wavefront (256 dims: two) at every number of heads."""
+    q, k, starts, ends = _qsa_case(rows, heads, dim, keys, dtype)
+    _check_qsa(ops.qsa_indexer_logits(q, k, starts.cuda(), ends.cuda()), q, k, starts, ends, math.sqrt(dim))
+
+
+@pytest.mark.parametrize('heads', [1, 2, 4, 8, 16, 32])
+@pytest.mark.parametrize('dim,dtype,odd', [(64, torch.bfloat16, 0), (64, torch.float16, 1), (128, torch.bfloat16, 1),
+                                           (128, torch.float16, 0), (256, torch.bfloat16, 0), (256, torch.float16, 1)])
+def test_qsa_indexer_logits_rows_far_apart(heads, dim, dtype, odd):
+    """Logit rows so far apart that a workgroup's rows pass 2^31 bytes; the columns past the keys stay as they are."""
+    rows, keys = 7, 1000 + 37 * odd
+    ld = (heads << 20) + 4 + odd
+    q, k, starts, ends = _qsa_case(rows, heads, dim, keys, dtype)
+    buf = torch.empty(rows, ld, device='cuda')
+    buf[:, keys:keys + 64] = 7.0
+    s, e = starts.cuda(), ends.cuda()
+    lib = ops._lib
+    lib.check(lib.lib().xt_qsa_indexer_logits(
+        q.data_ptr(), q.stride(0), q.stride(1), rows, heads, dim, k.data_ptr(), k.stride(0), keys, s.data_ptr(),
+        e.data_ptr(), 1.5, lib.XT_DTYPE_BF16 if dtype == torch.bfloat16 else lib.XT_DTYPE_F16, buf.data_ptr(), ld,
+        torch.cuda.current_stream().cuda_stream), 'qsa_indexer_logits')
+    _check_qsa(buf[:, :keys], q, k, starts, ends, 1.5)
+    assert (buf[:, keys:keys + 64] == 7.0).all()
+
+
 @pytest.mark.parametrize('rows,prefix', [(352, 380000), (1000, 100000), (64, 8192), (4096, 30000), (37, 500000)])
 def test_qsa_indexer_logits_reference_cases(rows, prefix):
     """The cases of tests/qsa_prefill_check.py:25-53: 4 heads x 128, compressed keys (ratio 4) up to the last row, each
