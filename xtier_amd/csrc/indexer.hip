@@ -252,7 +252,8 @@ __device__ inline void map_set(uint32_t* map, uint32_t col, uint32_t shift) {
 // and the histogram starts after the whole row has arrived.
 // PACK: only the top 16 bits of a key stay in registers, two keys to one, so a CU holds two rows of 98304 columns (one
 // loads while the other computes) or one of 196608; the candidates' keys are read from the row again, and a list
-// overflow reads the row for each of its three passes. 352 rows x 95088 columns: 49.3 us (2.7 TB/s) against 63.4 us for
+// overflow reads the row for each of its three passes, four chunks in flight (352 rows x 95088 values within a sixteenth
+// of each other: 280 us one by one, 255 us; 237 us with whole keys). 352 rows x 95088 columns: 49.3 us (2.7 TB/s) against 63.4 us for
 // one row of whole keys per CU, 49000 columns 26.2 us against 35.1 us; 32 rows x 131072 columns 40.6 us against 205.7 us
 // for the streaming kernel. Up to one row per CU the whole keys are faster (more wavefronts per row: 26.7 us at 95088
 // columns), past it two rows to a CU are (270 rows: 42.5 us against 55.7 us).
@@ -396,13 +397,18 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
     // f(i, the whole keys of chunk i): from the registers, or (PACK, not unrolled) from the row again
     const auto for_chunks = [&](auto f) {
       if constexpr (PACK) {
+        constexpr int kOnce = 4;   // chunks in flight
 #pragma unroll 1
-        for (int i = 0; i < CH; ++i) {
-          uint32_t k4[4];
-          load(i, k4);
+        for (int i = 0; i < CH; i += kOnce) {
+          uint32_t k4[kOnce][4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) k4[e] = convert(i, e, k4[e]);
-          f(i, k4);
+          for (int u = 0; u < kOnce; ++u) load(i + u, k4[u]);
+#pragma unroll
+          for (int u = 0; u < kOnce; ++u) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) k4[u][e] = convert(i + u, e, k4[u][e]);
+            f(i + u, k4[u]);
+          }
         }
       } else {
 #pragma unroll
