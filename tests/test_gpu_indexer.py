@@ -96,6 +96,16 @@ def test_topk_rows_off_16_byte_alignment(rows, cols, skip):
     assert np.array_equal(got[-1:], ref.topk_rows(x[skip:].view(rows, cols)[-1:].numpy(), 2048))
 
 
+@pytest.mark.parametrize('cols', [1, 3, 4, 255, 1000])
+def test_topk_rows_short_rows_of_many(cols):
+    """More than two rows per CU: rows of any length take the register forms."""
+    g = torch.Generator().manual_seed(cols)
+    x = torch.round(torch.randn(520, cols, generator=g) * 64) / 64
+    x[1], x[2, ::2], x[3] = -math.inf, math.nan, 0.0
+    for k in (1, 300):
+        assert np.array_equal(ops.topk_rows(x.cuda(), k).cpu().numpy(), ref.topk_rows(x.numpy(), k))
+
+
 def test_topk_rows_empty_rows():
     x = torch.randn(3, 8, device='cuda')[:, :0]          # rows of no column: nothing is read, every entry is -1
     assert np.array_equal(ops.topk_rows(x, 5).cpu().numpy(), np.full((3, 5), -1, np.int32))

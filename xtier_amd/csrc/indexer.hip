@@ -1129,14 +1129,21 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
   if (ld < cols || out_ld < topk) return fail(XT_EINVAL, "%s: row strides shorter than the rows", what);
   // empty rows stream, reading nothing, and come out all -1
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // short rows stream: the 8192-bucket histogram costs more than the passes it saves (601 columns: 6.3 us against 9.2 us;
-  // 4093: 11.6 us against 8.8 us at 32 rows, 17.2 us against 10.1 us at 352)
-  if (cols > (rows > device_cus() ? 1024 : 2048) && cols <= kTopkRegMax) {
+  // Short rows stream while every row is on the CUs at once (two workgroups to a CU): the 8192-bucket histogram costs more
+  // than the passes it saves. 512 keys, streamed / in registers: up to 2048 columns with at most a row per CU (32 rows x
+  // 1000 columns 6.4 / 8.8 us, x 2048 8.0 / 8.8 us), up to 1024 with two (512 x 1000 9.3 / 9.8 us; 257 x 1300 9.4 / 9.4
+  // us). Past that the register form's eight workgroups to a CU win at any length (513 rows x 400 11.5 / 10.3 us, 1024
+  // x 1000 16.6 / 12.4 us).
+  const int streamed = rows <= device_cus() ? 2048 : rows <= 2 * device_cus() ? 1024 : 0;
+  if (cols > streamed && cols <= kTopkRegMax) {
     const auto go = [&](auto kernel, int threads) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3((unsigned)threads), 0, st, x, ld, cols, topk, out, out_ld);
     };
     const bool al = cols % 4 == 0;
-    const bool many = rows > device_cus();   // past one round at one workgroup per CU: two packed ones share a CU
+    // past one round at one workgroup per CU two packed rows share a CU (whole / packed: 257 rows x 20000 columns 22.5 /
+    // 19.8 us, x 98304 53.7 / 44.1; 520 x 65536 59.2 / 55.9; 2048 x 32768 105 / 81; up to 16384 columns whole keys fit
+    // twice or more often as they are)
+    const bool many = rows > device_cus();
 #define XT_TOPK(TH, CH, PACK, RULE)                                                                                  \
   if (cols <= 4 * TH * CH && (RULE)) {                                                                               \
     al ? go(topk_rows_reg_kernel<TH, CH, true, PACK>, TH) : go(topk_rows_reg_kernel<TH, CH, false, PACK>, TH);       \
