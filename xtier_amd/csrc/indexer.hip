@@ -258,8 +258,8 @@ __device__ inline void map_set(uint32_t* map, uint32_t col, uint32_t shift) {
 // for the streaming kernel. Up to one row per CU the whole keys are faster (more wavefronts per row: 26.7 us at 95088
 // columns), past it two rows to a CU are (270 rows: 42.5 us against 55.7 us).
 template <int TH, int CH, bool ALIGNED4, bool PACK>
-__global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(const float* x, int64_t ld, int cols,
-                                                                          int topk, int32_t* out, int64_t out_ld) {
+__global__ __launch_bounds__(TH, TH > 256 && CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(
+    const float* x, int64_t ld, int cols, int topk, int32_t* out, int64_t out_ld) {
   constexpr int NW = TH / 64;
   constexpr int MAPW = TH * CH / 4;         // words per map
   // one list of keys and one of columns per wavefront fill the 32 KB histogram
@@ -397,7 +397,9 @@ __global__ __launch_bounds__(TH, CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(cons
     // f(i, the whole keys of chunk i): from the registers, or (PACK, not unrolled) from the row again
     const auto for_chunks = [&](auto f) {
       if constexpr (PACK) {
-        constexpr int kOnce = 4;   // chunks in flight
+        // chunks in flight (rows of other lengths load their last chunks element by element: one, since four cost the
+        // whole form 1 %)
+        constexpr int kOnce = ALIGNED4 ? 4 : 1;
 #pragma unroll 1
         for (int i = 0; i < CH; i += kOnce) {
           uint32_t k4[kOnce][4];
@@ -1132,7 +1134,7 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
   // Short rows stream while every row is on the CUs at once (two workgroups to a CU): the 8192-bucket histogram costs more
   // than the passes it saves. 512 keys, streamed / in registers: up to 2048 columns with at most a row per CU (32 rows x
   // 1000 columns 6.4 / 8.8 us, x 2048 8.0 / 8.8 us), up to 1024 with two (512 x 1000 9.3 / 9.8 us; 257 x 1300 9.4 / 9.4
-  // us). Past that the register form's eight workgroups to a CU win at any length (513 rows x 400 11.5 / 10.3 us, 1024
+  // us). Past that the register form's four workgroups to a CU win at any length (513 rows x 400 11.5 / 10.3 us, 1024
   // x 1000 16.6 / 12.4 us).
   const int streamed = rows <= device_cus() ? 2048 : rows <= 2 * device_cus() ? 1024 : 0;
   if (cols > streamed && cols <= kTopkRegMax) {
