@@ -484,7 +484,7 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
         }
       }
     }
-    if (++sub == subs) {   // the block is complete: max(round(c x)) = round(c max(x)) for c > 0 (else mr is -inf, unused)
+    if (++sub == subs) {   // the block is complete: max(round(c x)) = round(c max(x)) for c > 0, else mr is unused
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const float v = swap32_max(a.c > 0.0f ? fmaxf(m[g], mr[g] * a.c) : m[g]);

@@ -2,16 +2,17 @@
 // selection that turns them into the int32 [rows, topk] position lists the attention kernels read.
 //
 //   QSA indexer logits (BF16 / FP16 q and k): logits[r, n] = sum_h ReLU(q[r, h] . k[n]) / score_scale, -inf outside
-//     the row's [start, end). v_mfma_f32_32x32x16_{bf16,f16}: A = 32 keys x 16 dims, B = 16 dims x (32 / H rows x H
-//     heads); ReLU and the head sum on the accumulators (H lanes apart within a row of 16 lanes); the division as a
-//     multiplication by 1 / score_scale.
+//     the row's [start, end). v_mfma_f32_32x32x16_{bf16,f16}: A = (32 / H rows x H heads) x 16 dims, B = 16 dims x 32
+//     keys staged in LDS; a lane holds one key and 16 (row, head) pairs, so ReLU and the head sum run on its
+//     accumulators (from 8 heads on with one exchange with the lane 32 apart); the division as a multiplication by
+//     1 / score_scale. Logit rows too far apart for 31-bit offsets take a kernel that reads the keys straight from L2.
 //   DSA logits (FP8 E4M3 q and k, an FP32 scale per key, FP32 head weights): logits[q, n] = sum_h w[q, h] ReLU(q_h .
 //     k_n) * k_scale[n], outside [ks, ke) 0 or -inf. v_mfma_f32_32x32x16_f16 on the E4M3 values converted exactly to
 //     FP16, with the heads as rows (A = 32 heads x 16 dims of one query, B = 16 dims x 32 keys): a lane then holds 16
 //     heads of one key, so the weighted head sum is 16 FMAs in the lane and one exchange with the lane 32 apart. (The
 //     FP8 MFMA rounds inside its 16-product sum, to about 2^-16 of the sum of magnitudes; the FP16 one sums the exact
-//     products to FP32 accuracy.) Keys come from a flat array or, for decode, from
-//     the paged cache (page = block x D E4M3 values, then block FP32 scales) through the block table.
+//     products to FP32 accuracy.) Keys come from a flat array or, for decode, from the paged cache (page = block x D
+//     E4M3 values, then block FP32 scales) through the block table.
 //   Top-k rows: per row the positions of the topk largest finite values, ascending (ties toward the lower position),
 //     -1 padded. One workgroup per row: a three-pass radix select over an order-preserving key finds the topk-th
 //     largest key T and how many keys equal to T are taken. Rows up to 196608 columns live in registers: the first
@@ -153,30 +154,29 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* x,
   for (int i = (int)k + tid; i < topk; i += kTopkThreads) o[i] = -1;
 }
 
-// Rows of at most kTopkRegMax columns: the row is read once into registers as order keys (a
-// non-finite value as key 0, which no finite value has; the smallest finite key is 0x00800000). Chunk i of thread t
-// holds columns 4 (TH i + t) .. + 3.
+// Rows of at most kTopkRegMax columns: the row is read once into registers as order keys (a non-finite value as key 0,
+// which no finite value has; the smallest finite key is 0x00800000). Chunk i of thread t holds columns 4 (TH i + t) ..
+// + 3.
 //   1. A histogram of the top 13 bits finds the bucket b0 that holds the topk-th largest key (counted as the row
-//      arrives when the loads need no branches).
-//   2. One pass over the registers classifies every key: a bucket above b0 is taken (bit e of byte
-//      TH i + t of the taken map, so byte j covers columns 4 j .. 4 j + 3), a key in b0 is a candidate,
-//      appended with its column to its wavefront's list in LDS.
-//   3. Two histograms over the candidates (bits 18..9, then 8..0, both over 1024 buckets) find the topk-th largest
-//      key T and how many keys equal to T are taken; the candidates above T join the taken map, those equal to T go
-//      to the tie map. When a wavefront's list overflows, the two histograms run over the registers instead and the
-//      maps are rewritten against T.
-//   4. Thread t turns bytes CH t .. CH (t + 1) - 1 of both maps (columns 4 CH t ..) into positions in column
-//      order: one block scan places them, and a key equal to T is written only while fewer than `remaining` of them
-//      come before it.
-// 1024 threads (four wavefronts per SIMD, 96 keys and 128 registers each) measured 67.5 us against 70.7 us for 512
-// threads of 192 keys on 352 rows x 95088 columns: the extra wavefronts hide more of the LDS-atomic and branch latency
+//      arrives).
+//   2. One pass over the registers classifies every key: one of a bucket above b0 is taken (bit e of byte TH i + t of
+//      the map, so byte j covers columns 4 j .. 4 j + 3), one of b0 is a candidate, appended with its column to its
+//      wavefront's list in LDS.
+//   3. Two histograms over the candidates (bits 18..9, then 8..0, both over 1024 buckets) find the topk-th largest key
+//      T and how many keys equal to T are taken; the candidates above T join the taken bits, those equal to T are ties
+//      (bits 4-7 of the map's bytes). When a wavefront's list overflows, the two histograms run over the whole row
+//      instead and the map is rewritten against T.
+//   4. Thread t turns bytes CH t .. CH (t + 1) - 1 of the map (columns 4 CH t ..) into positions in column order: one
+//      block scan places them, and a key equal to T is written only while fewer than `remaining` of them come before
+//      it.
 //
 // A workgroup of TH threads holds CH chunks, 4 TH CH columns, and every chunk costs its share of each pass whether the
 // row fills it or not, so a row takes the smallest form that holds it (xt_topk_rows). Measured per call at 512 keys,
-// the form of 98304 columns -> the smallest: 4096 columns 26.7 us -> 8.3 us (1 row), 54.4 us -> 10.0 us (352 rows,
-// several workgroups to a CU); 32768 columns 26.4 us -> 15.4 us (32 rows).
-// a 16-byte load of dword alignment, all that these loads need: rows of any stride take the register forms (32 rows x
-// 32767 columns 59.6 us -> 15.4 us, 352 x 95087 254 us -> 46 us, against streaming them)
+// the form of 98304 columns -> the smallest: 4096 columns 26.7 us -> 8.4 us (1 row), 54.4 us -> 9.7 us (352 rows,
+// several workgroups to a CU); 32768 columns 26.4 us -> 14.6 us (32 rows). Bound: LDS atomics of the histogram, then
+// the classification and two block scans in a row, on as many CUs as there are rows.
+// A 16-byte load of dword alignment is all that these loads need: rows of any stride take the register forms (32 rows x
+// 32767 columns 59.6 us -> 14.6 us, 352 x 95087 254 us -> 46 us, against streaming them).
 typedef float4_t float4_dw_t __attribute__((aligned(4)));
 constexpr int kTopkRegMax = 4 * 1024 * 48;   // columns of the largest form
 
@@ -240,7 +240,7 @@ __device__ inline uint32_t pick_bucket(const uint32_t* h, uint32_t& remaining, u
   return bucket;
 }
 
-// Sets the bit of column `col` (plus `shift`: 4 for the ties) in the byte map (byte col / 4) with a word-wide LDS atomic.
+// Sets the bit of column `col` (plus `shift`: 4 for the ties) in the byte map (byte col / 4): a word-wide LDS atomic.
 __device__ inline void map_set(uint32_t* map, uint32_t col, uint32_t shift) {
   const uint32_t byte = col >> 2;
   atomicOr(&map[byte >> 2], 1u << (8u * (byte & 3u) + (col & 3u) + shift));
@@ -252,11 +252,11 @@ __device__ inline void map_set(uint32_t* map, uint32_t col, uint32_t shift) {
 // and the histogram starts after the whole row has arrived.
 // PACK: only the top 16 bits of a key stay in registers, two keys to one, so a CU holds two rows of 98304 columns (one
 // loads while the other computes) or one of 196608; the candidates' keys are read from the row again, and a list
-// overflow reads the row for each of its three passes, four chunks in flight (352 rows x 95088 values within a sixteenth
-// of each other: 280 us one by one, 255 us; 237 us with whole keys). 352 rows x 95088 columns: 49.3 us (2.7 TB/s) against 63.4 us for
-// one row of whole keys per CU, 49000 columns 26.2 us against 35.1 us; 32 rows x 131072 columns 40.6 us against 205.7 us
-// for the streaming kernel. Up to one row per CU the whole keys are faster (more wavefronts per row: 26.7 us at 95088
-// columns), past it two rows to a CU are (270 rows: 42.5 us against 55.7 us).
+// overflow reads the row for each of its three passes, four chunks in flight. 352 rows x 95088 columns: 46.9 us (2.9
+// TB/s) against 63.4 us for one row of whole keys per CU; 32 rows x 131072 columns 40.6 us against 205.7 us for the
+// streaming kernel. The price is the overflow: 352 rows x 95088 values within a sixteenth of each other take 255 us
+// (280 us one chunk at a time) against 237 us with whole keys. Up to one row per CU whole keys are as fast where the
+// lists hold (95088 columns, 1 row 25.4 us, packed 25.5) and faster where they overflow (111 us, packed 127).
 template <int TH, int CH, bool ALIGNED4, bool PACK>
 __global__ __launch_bounds__(TH, TH > 256 && CH <= 8 ? 8 : 4) void topk_rows_reg_kernel(
     const float* x, int64_t ld, int cols, int topk, int32_t* out, int64_t out_ld) {
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(TH, TH > 256 && CH <= 8 ? 8 : 4) void topk_rows_reg
       if constexpr (PACK) {
         key[i][0] = __builtin_amdgcn_perm(k4[1], k4[0], 0x07060302u);
         key[i][1] = __builtin_amdgcn_perm(k4[3], k4[2], 0x07060302u);
-        asm volatile("" : "+v"(key[i][0]), "+v"(key[i][1]));   // packed here: sunk to their uses, the four keys would stay
+        asm volatile("" : "+v"(key[i][0]), "+v"(key[i][1]));   // packed here: else the four keys stay to their uses
       }
     }
   }
@@ -667,16 +667,20 @@ __global__ __launch_bounds__(64 * kQsaWaves) void qsa_logits_kernel(const QsaArg
   }
 }
 
-// Keys through LDS: a workgroup is 4 wavefronts x G column groups of 32 / H rows over keys_per_wg keys, S keys at a time
-// staged once for all its 128 G (row, head) columns. Queries are the MFMA rows (A: column j of a group; B: keys), so C
-// lane (key kb + j, columns 8 (r / 4) + 4 h + r % 4) holds whole rows for H <= 4 and half rows, exchanged with the lane
-// 32 apart, for H >= 8. The next stage's loads are issued before this stage's stores and the stores carry no branch
-// (rows and keys past the end have offsets past the buffer's range, which drops them), so the wait for those loads does
-// not wait for the stores behind them. The stores are non-temporal: a row's logits are read once, by the selection, and
-// are written in 512-byte pieces of 128 rows at a time (60.5 us -> 52.4 us). Bound: HBM, the FP32 logits written, with
-// the matrix product and the head sum beside it (from 8 heads on they are the larger part). 352 rows x 95088 keys, 4
-// heads x 128: 52.4 us (3.0 TB/s) against 91.8 us for the kernel above, whose wavefronts each read the keys from L2 and
-// wait for their stores with them; 352 x 65536: 8 heads 128 -> 61 us, 16 heads 261 -> 99, 32 heads 590 -> 188.
+// Keys through LDS: a workgroup is 4 wavefronts x G column groups of 32 / H rows over keys_per_wg keys, S keys at a
+// time staged once for all its 128 G (row, head) columns. Queries are the MFMA rows (A: column j of a group; B: keys),
+// so C lane (key kb + j, columns 8 (r / 4) + 4 h + r % 4) holds whole rows for H <= 4 and half rows, exchanged with the
+// lane 32 apart, for H >= 8. The next stage's loads are issued before this stage's stores and the stores carry no
+// branch (rows and keys past the end have offsets past the buffer's range, which drops them), so the wait for those
+// loads does not wait for the stores behind them. Bound: HBM, the FP32 logits written, with the matrix product and the
+// head sum beside it (from 8 heads on they are the larger part). 352 rows x 95088 keys, 4 heads x 128: 50.4 us (3.1
+// TB/s) against 91.8 us for the kernel above, whose wavefronts each read the keys from L2 and wait for their stores
+// with them; 352 x 65536: 8 heads 128 -> 61 us, 16 heads 261 -> 99, 32 heads 590 -> 188.
+// The stores are non-temporal: the logits alone take 50.4 us in place of 60.5 at 352 x 95088. With the selection of
+// 2048 positions behind them (4 heads, plain -> non-temporal): 352 x 4100 keys 23.0 -> 21.6 us, 352 x 32768 48.3 ->
+// 47.5, 32 x 65536 29.7 -> 29.3; but 32 x 4100 13.9 -> 14.4, and from about 60 MB of logits on the selection, which
+// then reads them from HBM, loses more than the stores gain (352 x 65536 78.3 -> 79.4, x 95088 104.5 -> 109.5; 512 x
+// 95088 129 -> 137).
 template <int NK, int G>
 constexpr int kQsaStage = (NK <= 8 ? 64 : 32) * (G == 4 ? 2 : 1);   // keys per stage
 
@@ -826,8 +830,8 @@ __global__ __launch_bounds__(64 * kQsaWaves, 2) void qsa_logits_lds_kernel(const
         }
 #pragma unroll
         for (int o = 0; o < kOut; ++o)
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[o]), rsrc, (int)(koff + (uint32_t)(g * kRowsG + first(o)) * row_step),
-                                              0, 2);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[o]), rsrc,
+                                              (int)(koff + (uint32_t)(g * kRowsG + first(o)) * row_step), 0, 2);
       }
     }
   }
@@ -863,10 +867,10 @@ struct DsaArgs {
 constexpr int kDsaWaves = 4;
 
 // The shapes the two kernels below do not take (query and weights past their registers, pages off the 32-key grid, rows
-// off 16-byte alignment). Workgroup = (4 query rows, one per wavefront, keys_per_wg keys); the wavefronts walk the same 32-key blocks, so a
-// block's key bytes are fetched once for the four rows. Per block and 32-head group, S = Q . K^T on 32x32x16 FP16
-// MFMAs of the converted E4M3 values (A = Q: lane (head l % 32, dims 16kk + 8 (l / 32) .. +7); B = K^T: lane (key
-// l % 32, same dims); C: lane (key column l % 32, heads 8 (r / 4) + 4 (l / 32) + r % 4)).
+// off 16-byte alignment). Workgroup = (4 query rows, one per wavefront, keys_per_wg keys); the wavefronts walk the same
+// 32-key blocks, so a block's key bytes are fetched once for the four rows. Per block and 32-head group, S = Q . K^T on
+// 32x32x16 FP16 MFMAs of the converted E4M3 values (A = Q: lane (head l % 32, dims 16kk + 8 (l / 32) .. +7); B = K^T:
+// lane (key l % 32, same dims); C: lane (key column l % 32, heads 8 (r / 4) + 4 (l / 32) + r % 4)).
 template <int NK>
 __global__ __launch_bounds__(64 * kDsaWaves) void dsa_logits_kernel(const DsaArgs a) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
@@ -1021,11 +1025,11 @@ __global__ __launch_bounds__(64 * kDsaWaves) void dsa_flat_kernel(const DsaArgs 
 // Paged keys whose pages hold a multiple of 32 keys (decode): one row per workgroup, `bpw` consecutive 32-key blocks
 // per wavefront, so a batch of a few rows still spreads over every CU. The row's query (as FP16) and head weights stay
 // in registers for the wavefront's whole range; a block's page is uniform, so the wavefront's table entries are one
-// vector load before the loop and a block's address is scalar. Bound: HBM, D + 4 bytes per key; a wavefront keeps one
-// block's loads in flight beyond the one it computes (two or three measured 21.3 us against 20.8). k-step kk covers dims h D/2 + 8 kk .. + 7 in both operands (not
-// 16 kk + 8 h), so a lane reads its half of a key's row as 16-byte pieces. Measured at 32 rows x 32 heads x 128, up to
-// 32768 keys each (16.6K in the mean, 69 MB): 20.8 us = 3.3 TB/s against 352 us for dsa_logits_kernel, which puts four rows in a workgroup
-// and 4096 keys in a wavefront's serial walk.
+// vector load before the loop and a block's address is scalar. k-step kk covers dims h D/2 + 8 kk .. + 7 in both
+// operands (not 16 kk + 8 h), so a lane reads its half of a key's row as 16-byte pieces. Bound: HBM, D + 4 bytes per
+// key; a wavefront keeps one block's loads in flight beyond the one it computes (two or three measured 21.3 us against
+// 20.8). 32 rows x 32 heads x 128, up to 32768 keys each (16.6K in the mean, 69 MB): 20.8 us = 3.3 TB/s against 352 us
+// for dsa_logits_kernel, which puts four rows in a workgroup and 4096 keys in a wavefront's serial walk.
 constexpr int kDsaAhead = 1;
 
 template <int NK, int G>
@@ -1095,7 +1099,8 @@ __global__ __launch_bounds__(64 * kDsaWaves) void dsa_paged_kernel(const DsaArgs
 #pragma unroll
     for (int s = 0; s < kDsaAhead; ++s)
       if (s < live_blocks) load(s, s);
-    // kDsaAhead + 1 blocks per trip, so every register slot is a constant; the trips before the last blocks test nothing
+    // kDsaAhead + 1 blocks per trip, so every register slot is a constant; the trips before the last blocks test
+    // nothing
     constexpr int S = kDsaAhead + 1;
     int i = 0;
     for (; i + S + kDsaAhead <= live_blocks; i += S) {
@@ -1131,20 +1136,20 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
   if (ld < cols || out_ld < topk) return fail(XT_EINVAL, "%s: row strides shorter than the rows", what);
   // empty rows stream, reading nothing, and come out all -1
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // Short rows stream while every row is on the CUs at once (two workgroups to a CU): the 8192-bucket histogram costs more
-  // than the passes it saves. 512 keys, streamed / in registers: up to 2048 columns with at most a row per CU (32 rows x
-  // 1000 columns 6.4 / 8.8 us, x 2048 8.0 / 8.8 us), up to 1024 with two (512 x 1000 9.3 / 9.8 us; 257 x 1300 9.4 / 9.4
-  // us). Past that the register form's four workgroups to a CU win at any length (513 rows x 400 11.5 / 10.3 us, 1024
-  // x 1000 16.6 / 12.4 us).
+  // Short rows stream while every row is on the CUs at once (two workgroups to a CU): the 8192-bucket histogram costs
+  // more than the passes it saves. 512 keys, streamed / in registers: up to 2048 columns with at most a row per CU (32
+  // rows x 1000 columns 6.4 / 8.8 us, x 2048 8.0 / 8.8 us), up to 1024 with two (512 x 1000 9.3 / 9.8 us; 257 x 1300
+  // 9.4 / 9.4 us). Past that the register form's four workgroups to a CU win at any length (513 rows x 400 11.5 / 10.3
+  // us, 1024 x 1000 16.6 / 12.4 us).
   const int streamed = rows <= device_cus() ? 2048 : rows <= 2 * device_cus() ? 1024 : 0;
   if (cols > streamed && cols <= kTopkRegMax) {
     const auto go = [&](auto kernel, int threads) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3((unsigned)threads), 0, st, x, ld, cols, topk, out, out_ld);
     };
     const bool al = cols % 4 == 0;
-    // past one round at one workgroup per CU two packed rows share a CU (whole / packed: 257 rows x 20000 columns 22.5 /
-    // 19.8 us, x 98304 53.7 / 44.1; 520 x 65536 59.2 / 55.9; 2048 x 32768 105 / 81; up to 16384 columns whole keys fit
-    // twice or more often as they are)
+    // past one round at one workgroup per CU two packed rows share a CU (whole / packed: 257 rows x 20000 columns 22.5
+    // / 19.8 us, x 98304 53.7 / 44.1; 520 x 65536 59.2 / 55.9; 2048 x 32768 105 / 81; up to 16384 columns whole keys
+    // fit twice or more often as they are)
     const bool many = rows > device_cus();
 #define XT_TOPK(TH, CH, PACK, RULE)                                                                                  \
   if (cols <= 4 * TH * CH && (RULE)) {                                                                               \
@@ -1152,7 +1157,8 @@ extern "C" int xt_topk_rows(const float* x, int64_t ld, int rows, int cols, int 
     return check_launch(what);                                                                                       \
   }
     XT_TOPK(256, 4, false, true) XT_TOPK(512, 4, false, true) XT_TOPK(1024, 4, false, true)
-    XT_TOPK(512, 16, true, many) XT_TOPK(1024, 8, false, true) XT_TOPK(512, 24, true, many) XT_TOPK(1024, 12, false, true)
+    XT_TOPK(512, 16, true, many) XT_TOPK(1024, 8, false, true) XT_TOPK(512, 24, true, many)
+    XT_TOPK(1024, 12, false, true)
     XT_TOPK(512, 32, true, many) XT_TOPK(1024, 16, false, true) XT_TOPK(512, 48, true, many)
     XT_TOPK(1024, 24, false, true) XT_TOPK(1024, 48, true, true)
 #undef XT_TOPK
@@ -1175,8 +1181,9 @@ static int qsa_per_cu() {
   return n;
 }
 
-// Rows too long for the LDS kernel's 31-bit offsets. The grid: row tiles x key chunks, the chunks sized so that the workgroups fit one round on the CUs (a second round
-// of a few workgroups would take as long as the first: 558 workgroups at 512 per round measured 116 us).
+// Rows too far apart for the LDS kernel's 31-bit offsets. The grid: row tiles x key chunks, the chunks sized so that
+// the workgroups fit one round on the CUs (a second round of a few workgroups would take as long as the first: 558
+// workgroups at 512 per round measured 116 us).
 template <int H, int NK, bool BF>
 static void qsa_go(QsaArgs a, int row_tiles, hipStream_t st) {
   const int64_t slots = (int64_t)device_cus() * qsa_per_cu<H, NK, BF>();

@@ -295,8 +295,8 @@ __device__ inline int64_t part_index(const MlaArgs& a, int64_t row, int split, i
   return ((((row * a.splits + split) * waves + wave) * 16 + k) * 64 + lane) * 8;
 }
 
-// TL: the per-wave timeline build (xt_mla_timeline) of each form, launched only while a stamp buffer is set, so the kernel
-// the serving path runs carries none of its instructions or registers.
+// TL: the per-wave timeline build (xt_mla_timeline) of each form, launched only while a stamp buffer is set, so the
+// kernel the serving path runs carries none of its instructions or registers.
 // PART: launches with whole waves of absent heads (heads <= 112) or with list lengths: a wave without a live head only
 // dequantizes, so the others have the matrix cores and the LDS to themselves, and a step without a valid key is
 // dequantized only. 64 heads: 1024 rows of 2048 keys (NVFP4) 576 us -> 431 us, 61 rows of 640 keys (V4, lists three
@@ -459,87 +459,88 @@ __global__ void __launch_bounds__(512) mla_kernel(const MlaArgs a) {
     if (step + 2 < a.steps) load_raw<F, TWO>(a, slots, step + 2, raw);
     const uint32_t valid = (uint32_t)__builtin_amdgcn_ballot_w64(lane < kMSteps &&
                                                                   entry_valid(slots[step * kMSteps + (lane & 31)]));
-    if (!PART || (wave_live && valid != 0u)) {
-    // S^T for the two 16-key tiles, one MFMA chain each. The K fragments (and LDS-resident query chunks) of chunk
-    // kk + kQAhead are read while the MFMAs of chunk kk run; scheduling barriers keep that order, so an MFMA does not
-    // wait for a read issued just before it.
-    // this lane's keys T(j) as bits 0..7: keys 4j .. 4j+3, then 16+4j .. 16+4j+3
-    const uint32_t vmask = ((valid >> (4 * j)) & 0xFu) | (((valid >> (16 + 4 * j)) & 0xFu) << 4);
-    // NVFP4: the global scale of each of those keys (of its cache; two caches may differ). Chunks below kLatC are the
-    // latent's: once they are summed, the accumulators are multiplied by the key's global scale, and the rope chunks
-    // (no global scale) add onto them.
-    uint32_t l1 = 0u;   // bit e: key e of T(j) is cache 1's
-    if constexpr (F == kNvfp4 && TWO) {
-      const uint32_t b =
-          (uint32_t)__builtin_amdgcn_ballot_w64(lane < kMSteps && slots[step * kMSteps + (lane & 31)] <= -2);
-      l1 = ((b >> (4 * j)) & 0xFu) | (((b >> (16 + 4 * j)) & 0xFu) << 4);
-    }
-    float4_t s[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
-    short8_t kf[kQC][2], qf[kQC];
-    auto read_chunk = [&](int kk) {
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-        kf[kk][tt] = *reinterpret_cast<const short8_t*>(kt + (16 * tt + hl) * kKRow<F> + 8 * j + 32 * kk);
-      qf[kk] = kk < kQR ? qb[kk < kQR ? kk : 0]
-                        : *reinterpret_cast<const short8_t*>(qs + ((kk - kQR) * kMHeads + 16 * wave + hl) * kQRow +
-                                                             8 * (j ^ ((hl >> 1) & 3)));
-    };
-#pragma unroll
-    for (int kk = 0; kk < kQAhead; ++kk) read_chunk(kk);
-#pragma unroll
-    for (int kk = 0; kk < kQC; ++kk) {
-      if (kk + kQAhead < kQC) read_chunk(kk + kQAhead);
-      __builtin_amdgcn_sched_barrier(0);
-      if (kk == kLatC) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s[e >> 2][e & 3] *= ((l1 >> e) & 1u) ? g1 : g0;
+    if (!PART || (wave_live && valid != 0u)) {   // absent heads and steps without a key: dequantized only
+      // S^T for the two 16-key tiles, one MFMA chain each. The K fragments (and LDS-resident query chunks) of chunk
+      // kk + kQAhead are read while the MFMAs of chunk kk run; scheduling barriers keep that order, so an MFMA does not
+      // wait for a read issued just before it.
+      // this lane's keys T(j) as bits 0..7: keys 4j .. 4j+3, then 16+4j .. 16+4j+3
+      const uint32_t vmask = ((valid >> (4 * j)) & 0xFu) | (((valid >> (16 + 4 * j)) & 0xFu) << 4);
+      // NVFP4: the global scale of each of those keys (of its cache; two caches may differ). Chunks below kLatC are the
+      // latent's: once they are summed, the accumulators are multiplied by the key's global scale, and the rope chunks
+      // (no global scale) add onto them.
+      uint32_t l1 = 0u;   // bit e: key e of T(j) is cache 1's
+      if constexpr (F == kNvfp4 && TWO) {
+        const uint32_t b =
+            (uint32_t)__builtin_amdgcn_ballot_w64(lane < kMSteps && slots[step * kMSteps + (lane & 31)] <= -2);
+        l1 = ((b >> (4 * j)) & 0xFu) | (((b >> (16 + 4 * j)) & 0xFu) << 4);
       }
+      float4_t s[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+      short8_t kf[kQC][2], qf[kQC];
+      auto read_chunk = [&](int kk) {
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-        s[tt] = kk >= kLatC ? mfma16<kFp8V4>(kf[kk][tt], qf[kk], s[tt]) : mfma16<F>(kf[kk][tt], qf[kk], s[tt]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    float sv[8];
+        for (int tt = 0; tt < 2; ++tt)
+          kf[kk][tt] = *reinterpret_cast<const short8_t*>(kt + (16 * tt + hl) * kKRow<F> + 8 * j + 32 * kk);
+        qf[kk] = kk < kQR ? qb[kk < kQR ? kk : 0]
+                          : *reinterpret_cast<const short8_t*>(qs + ((kk - kQR) * kMHeads + 16 * wave + hl) * kQRow +
+                                                               8 * (j ^ ((hl >> 1) & 3)));
+      };
 #pragma unroll
-    for (int e = 0; e < 8; ++e) sv[e] = ((vmask >> e) & 1u) ? s[e >> 2][e & 3] * smul : -__builtin_inff();
-    // online softmax of head hl over keys T(j), lazy rescale
-    float mt = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
-    mt = max4_lanes16(mt);
-    if (__builtin_amdgcn_ballot_w64(mt > m + kRescaleM)) {
-      const float m_new = (mt > m + kRescaleM) ? mt : m;
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-      l *= alpha;
+      for (int kk = 0; kk < kQAhead; ++kk) read_chunk(kk);
 #pragma unroll
-      for (int i = 0; i < 32; ++i) acc[i] *= alpha;
-      m = m_new;
-    }
-    const float m_use = (m == -__builtin_inff()) ? 0.0f : m;
-    short8_t pb;
-    float psum = 0.0f;
+      for (int kk = 0; kk < kQC; ++kk) {
+        if (kk + kQAhead < kQC) read_chunk(kk + kQAhead);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kk == kLatC) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float p = __builtin_amdgcn_exp2f(sv[e] - m_use);
-      psum += p;
-      if constexpr (F == kNvfp4)
-        pb[e] = __builtin_bit_cast(short, (_Float16)(TWO ? p * ginv * (((l1 >> e) & 1u) ? g1 : g0) : p));
-      else
-        pb[e] = __builtin_bit_cast(short, (__bf16)p);
-    }
-    l += psum;
-    // O^T += V^T . P^T over the 32 dim tiles, V^T read from the K tile with transposing reads: in each 16-lane group
-    // lane L addresses key 4j + L/4, dims 16 dt + 4 (L % 4) .. +3, and lane i receives dim 16 dt + i of keys 4j .. 4j+3
-    // (then 16 + 4j .. from 16 rows further)
-    typedef short short4_t __attribute__((ext_vector_type(4)));
-    const uint16_t* vr = kt + (4 * j + (hl >> 2)) * kKRow<F> + 4 * (hl & 3);
+          for (int e = 0; e < 8; ++e) s[e >> 2][e & 3] *= ((l1 >> e) & 1u) ? g1 : g0;
+        }
 #pragma unroll
-    for (int dt = 0; dt < 32; ++dt) {
-      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) short4_t*)(vr + 16 * dt));
-      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) short4_t*)(vr + 16 * kKRow<F> + 16 * dt));
-      const short8_t av = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      acc[dt] = mfma16<F>(av, pb, acc[dt]);
-    }
+        for (int tt = 0; tt < 2; ++tt)
+          s[tt] = kk >= kLatC ? mfma16<kFp8V4>(kf[kk][tt], qf[kk], s[tt]) : mfma16<F>(kf[kk][tt], qf[kk], s[tt]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float sv[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sv[e] = ((vmask >> e) & 1u) ? s[e >> 2][e & 3] * smul : -__builtin_inff();
+      // online softmax of head hl over keys T(j), lazy rescale
+      float mt = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])),
+                       fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
+      mt = max4_lanes16(mt);
+      if (__builtin_amdgcn_ballot_w64(mt > m + kRescaleM)) {
+        const float m_new = (mt > m + kRescaleM) ? mt : m;
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        l *= alpha;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) acc[i] *= alpha;
+        m = m_new;
+      }
+      const float m_use = (m == -__builtin_inff()) ? 0.0f : m;
+      short8_t pb;
+      float psum = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float p = __builtin_amdgcn_exp2f(sv[e] - m_use);
+        psum += p;
+        if constexpr (F == kNvfp4)
+          pb[e] = __builtin_bit_cast(short, (_Float16)(TWO ? p * ginv * (((l1 >> e) & 1u) ? g1 : g0) : p));
+        else
+          pb[e] = __builtin_bit_cast(short, (__bf16)p);
+      }
+      l += psum;
+      // O^T += V^T . P^T over the 32 dim tiles, V^T read from the K tile with transposing reads: in each 16-lane group
+      // lane L addresses key 4j + L/4, dims 16 dt + 4 (L % 4) .. +3, and lane i receives dim 16 dt + i of keys 4j ..
+      // 4j+3 (then 16 + 4j .. from 16 rows further)
+      typedef short short4_t __attribute__((ext_vector_type(4)));
+      const uint16_t* vr = kt + (4 * j + (hl >> 2)) * kKRow<F> + 4 * (hl & 3);
+#pragma unroll
+      for (int dt = 0; dt < 32; ++dt) {
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) short4_t*)(vr + 16 * dt));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) short4_t*)(vr + 16 * kKRow<F> + 16 * dt));
+        const short8_t av = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        acc[dt] = mfma16<F>(av, pb, acc[dt]);
+      }
     }
     __syncthreads();
   }
@@ -576,8 +577,9 @@ __global__ void __launch_bounds__(512) mla_kernel(const MlaArgs a) {
     return;
   }
   // 2. the split's output normalized by its own sum (NVFP4: FP16, a convex combination of e2m1 * e4m3 values, so at
-  //    most 2688 in magnitude whatever g; V4: FP32) plus its max and sum; a second launch merges the splits. The partials are stored in the accumulators'
-  //    lane order (part_index), so every store of a wave writes one contiguous run.
+  //    most 2688 in magnitude whatever g; V4: FP32) plus its max and sum; a second launch merges the splits. The
+  //    partials are stored in the accumulators' lane order (part_index), so every store of a wave writes one contiguous
+  //    run.
   if (16 * wave >= a.heads) return;   // a wave without live heads has no partials (heads pad to whole waves only)
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;   // NVFP4: without g (the merge applies it)
   const int64_t pbase = part_index(a, row, split, wave, 0, lane);
