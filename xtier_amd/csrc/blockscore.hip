@@ -600,15 +600,30 @@ int score_common(const char* what, ScoreArgs& a, int dim, int q_dtype, const voi
 
 template <int NK, bool BF>
 int decode_dispatch(int T, const ScoreArgs& a, dim3 grid, hipStream_t st) {
-  if (a.heads <= 32 / NK) {   // the block-diagonal query fits the MFMA's rows
-    switch (T) {
-      case 1: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 1, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
-      case 2: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 2, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
-      case 4: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 4, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
-      case 8: hipLaunchKernelGGL((decode_scores_few_kernel<NK, 8, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
-      default: return XT_EUNSUPPORTED;
+  // The block-diagonal query fits the MFMA's rows. At 64 dims a block of 32 or 64 keys has fewer products than its
+  // reductions over the lanes, one per head, cost (heads x requests x keys, block size: this kernel / the other): 4 x 64
+  // x 32768, 32: 41.9 / 36.2 us; 4 x 16 x 4096, 64: 4.5 / 4.2; but 4 x 64 x 32768, 128: 36.2 / 44.4. At 128 dims it is
+  // ahead from 32 keys on (4 x 64 x 32768, 32: 49.8 / 50.1 us, 64: 48.4 / 49.3, 128: 52.8 / 60.0).
+  if (a.heads <= 32 / NK) {
+    const dim3 block(64 * kScoreWaves);
+    if constexpr (NK > 4) {
+      if (T == 1) {
+        hipLaunchKernelGGL((decode_scores_few_kernel<NK, 1, BF>), grid, block, 0, st, a);
+        return XT_OK;
+      }
+      if (T == 2) {
+        hipLaunchKernelGGL((decode_scores_few_kernel<NK, 2, BF>), grid, block, 0, st, a);
+        return XT_OK;
+      }
     }
-    return XT_OK;
+    if (T == 4) {
+      hipLaunchKernelGGL((decode_scores_few_kernel<NK, 4, BF>), grid, block, 0, st, a);
+      return XT_OK;
+    }
+    if (T == 8) {
+      hipLaunchKernelGGL((decode_scores_few_kernel<NK, 8, BF>), grid, block, 0, st, a);
+      return XT_OK;
+    }
   }
   switch (T) {
     case 1: hipLaunchKernelGGL((decode_scores_kernel<NK, 1, BF>), grid, dim3(64 * kScoreWaves), 0, st, a); break;
