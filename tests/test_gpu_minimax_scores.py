@@ -171,6 +171,16 @@ def test_prefill_scores_many_row_tiles(prefix, ext, dim, bs, heads, q_dtype):
     test_prefill_scores(prefix, ext, dim, bs, heads, q_dtype)
 
 
+@pytest.mark.parametrize('dim', [64, 128, 256])
+@pytest.mark.parametrize('bs,heads,width', [(32, 1, 16384), (32, 4, 17280), (64, 3, 16384), (64, 2, 35840)])
+def test_prefill_scores_blocks_shorter_than_a_chunk(monkeypatch, dim, bs, heads, width):
+    """Blocks that end inside a staged chunk of keys: ranges of whole chunks, and ranges (9 blocks, by the table's width)
+    and sequences that end inside one."""
+    mapping = _mapping
+    monkeypatch.setitem(globals(), '_mapping', lambda seq_lens, g: mapping(seq_lens, g, width))
+    test_prefill_scores([1000, 37, 0], [333, 95, 64], dim, bs, heads, torch.bfloat16 if bs == 32 else torch.float16)
+
+
 @pytest.mark.parametrize('factor', [-1.0, 0.0])
 def test_prefill_scores_with_a_factor_that_is_not_positive(factor):
     """The maximum is of the scaled values, so a negative factor takes the smallest product."""

@@ -229,9 +229,9 @@ __global__ __launch_bounds__(64 * kScoreWaves) void decode_scores_kernel(const S
 // unscaled key tile (one conversion per two values), and C holds, for one key per lane, the partial dot product of
 // every head and of the lane half's NK / 2 blocks, so the block scales enter as one FMA per (head, block) in FP32
 // (E4M3 values, exact). The kernel above multiplies every key value by its scale and spends its columns past `heads`
-// on nothing. Work split as above; the next block's slots are looked up behind the current block's loads. Bound: HBM, 76
-// bytes per key at 128 dims. 32 requests x 32768 keys, 4 heads: 20.8 us (3.8 TB/s) against 28.4 us for the kernel above
-// (22.1 us at 152 registers, three wavefronts per SIMD, hence the four in the launch bounds at up to 4 tiles).
+// on nothing. Work split as above; the next block's slots are looked up behind the current block's loads. Bound: HBM,
+// 76 bytes per key at 128 dims. 32 requests x 32768 keys, 4 heads: 20.8 us (3.8 TB/s) against 28.4 us for the kernel
+// above (22.1 us at 152 registers, three wavefronts per SIMD, hence the four in the launch bounds at up to 4 tiles).
 // A lane half's NK / 2 scale bytes, as loaded and as FP32.
 template <int NK>
 using ScaleWord = std::conditional_t<NK == 4, uint16_t, std::conditional_t<NK == 8, uint32_t, uint64_t>>;
@@ -357,20 +357,23 @@ __global__ __launch_bounds__(64 * kScoreWaves, (kFewWaves<NK, T>)) void decode_s
 // Prefill: grid (row tile x block range, request b, head group of HPW heads); a workgroup covers R = 128 G / HPW query
 // rows of request b and one range of chunk_blocks blocks (the per-block results are independent, so ranges split a
 // long prompt's work over many workgroups). Column j of wavefront w's column group g is (row (32 / HPW)(G w + g) +
-// j / HPW, head j % HPW). Key chunks of S = min(block_size, kStageKeys) positions are staged as 16-bit values in LDS
-// by the whole workgroup (two threads per key, once for its 128 G columns), then each wavefront runs its G column
-// groups over them. Two LDS stages: while one is computed on, the next chunk's payload and scales are in flight to
-// registers and the slots of the one after are being looked up, and one barrier per chunk suffices. Chunks wholly at
-// or below every row's position skip the causal test and scale once after the maximum (c > 0: the maximum commutes
-// with the rounding of the product).
-// Bound: the matrix cores, with the staging's conversions and LDS reads beside them, so G = 4 shares each staged key and
-// each LDS read among twice the columns. 4096 rows x 4 heads against 65536 keys at 128 dims (266 GFLOP): 235 us (1130
-// TFLOP/s) against 400 us for one LDS stage, G = 2 and a 64-bit division per staged piece.
+// j / HPW, head j % HPW). Key chunks of SK = kStageKeys positions are staged as 16-bit values in LDS by the whole
+// workgroup (two threads per key, once for its 128 G columns), then each wavefront runs its G column groups over them.
+// SHORT: blocks shorter than a chunk, which ends them tile by tile; a chunk per block, 32 keys, had left three quarters
+// of the threads idle while staging and made 64 dims slower than one LDS stage (4 heads x 8192 rows against 38192 keys
+// in blocks of 32: 466 us, 352 us now; 128 dims 510 us, 446 us).
+// Two LDS stages: while one is computed on, the next chunk's payload and scales are in flight to registers and the
+// slots of the one after are being looked up, and one barrier per chunk suffices. Chunks wholly at or below every row's
+// position skip the causal test and scale once after the maximum (c > 0: the maximum commutes with the rounding of the
+// product).
+// Bound: the matrix cores, with the staging's conversions and LDS reads beside them, so G = 4 shares each staged key
+// and each LDS read among twice the columns. 4096 rows x 4 heads against 65536 keys at 128 dims (266 GFLOP): 235 us
+// (1130 TFLOP/s) against 400 us for one LDS stage, G = 2 and a 64-bit division per staged piece.
 
 template <int NK>
 constexpr int kStageKeys = NK <= 8 ? 128 : 64;
 
-template <int NK, int HPW, int G, bool BF>
+template <int NK, int HPW, int G, bool BF, bool SHORT>
 __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(const ScoreArgs a) {
   constexpr int D = 16 * NK;
   constexpr int ROW_U32 = D / 2 + 4;          // LDS row: D 16-bit values + 16 bytes of padding
@@ -395,9 +398,10 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
   const int64_t blk_lo = (int64_t)chunk * a.chunk_blocks, blk_hi = min(wg_blocks, blk_lo + a.chunk_blocks);
   if (blk_lo >= wg_blocks) return;   // uniform: before every barrier
   const bool wide_r2t = a.wide & kWideR2t;
-  const int S = bs < SK ? bs : SK;
-  const int subs = bs / S;                                // chunks per block
-  const int n_chunks = (int)(blk_hi - blk_lo) * subs;
+  const int S = SHORT ? SK : bs < SK ? bs : SK;
+  const int parts = bs / (SHORT ? 32 : S);                // 32-key tiles or chunks per block
+  const int keys = (int)(blk_hi - blk_lo) * bs;
+  const int n_chunks = SHORT ? (keys + S - 1) / S : (int)(blk_hi - blk_lo) * parts;
   const int64_t pos_lo = blk_lo * bs;                     // first position of the range
   const int64_t r2t_row = sid * a.r2t_stride;
   // staging: thread 2 key + half takes that half of the key's dims
@@ -434,13 +438,27 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
     for (int kk = 0; kk < NK; ++kk)
       qv[g][kk] = live ? *reinterpret_cast<const u32x4_t*>(qp + 8 * kk) : u32x4_t{0, 0, 0, 0};
   }
-  // chunks before this one are at or below every row's position and below seq_len, whole
-  const int64_t whole = a.c > 0.0f ? max((int64_t)0, min(pre + row0 + 1, seq) - pos_lo) / S : 0;
+  // chunks (SHORT: tiles) before this one are at or below every row's position and below seq_len, whole
+  const int64_t whole = a.c > 0.0f ? max((int64_t)0, min(pre + row0 + 1, seq) - pos_lo) / (SHORT ? 32 : S) : 0;
   load_raw(slot_next);
   slot_next = slot_at(1);
   float m[G], mr[G];   // scaled maxima of masked chunks, raw maxima of unmasked ones
 #pragma unroll
   for (int g = 0; g < G; ++g) m[g] = mr[g] = -__builtin_inff();
+  // The block is complete: max(round(c x)) = round(c max(x)) for c > 0, else mr is unused. (As a lambda it took registers
+  // from the long form's loop, 1 %.)
+#define XT_BLOCK_DONE                                                                                                \
+  do {                                                                                                               \
+    _Pragma("unroll") for (int g = 0; g < G; ++g) {                                                                  \
+      const float v = swap32_max(a.c > 0.0f ? fmaxf(m[g], mr[g] * a.c) : m[g]);                                      \
+      const int64_t row = row0 + RG * (G * wave + g) + j / HPW;                                                      \
+      if (h == 0 && bi < nblk[g])                                                                                    \
+        store_score(a, (int64_t)head * a.s_hs + (q0 + row) * a.s_ns + (blk_lo + bi) * a.s_ks, v);                    \
+      m[g] = mr[g] = -__builtin_inff();                                                                              \
+    }                                                                                                                \
+    sub = 0;                                                                                                         \
+    ++bi;                                                                                                            \
+  } while (0)
   for (int n = 0, sub = 0, bi = 0; n < n_chunks; ++n) {
     uint32_t* buf = lds[n & 1];
     if (stager) {
@@ -456,8 +474,10 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
       slot_next = slot_at(n + 2);
     }
     __syncthreads();   // chunk n is staged; every wavefront is past chunk n - 1, whose buffer chunk n + 1 takes
-    const bool unmasked = n < whole;
-    for (int t = 0; t < S / 32; ++t) {
+    const int tiles32 = (SHORT ? min(S, keys - n * S) : S) / 32;
+    bool unmasked = n < whole;
+    for (int t = 0; t < tiles32; ++t) {
+      if (SHORT) unmasked = n * (SK / 32) + t < whole;
       float16_t s[G];
 #pragma unroll
       for (int g = 0; g < G; ++g) s[g] = float16_t{};
@@ -483,20 +503,11 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
             m[g] = fmaxf(m[g], 8 * (r >> 2) + (r & 3) <= lim ? s[g][r] * a.c : -__builtin_inff());
         }
       }
+      if (SHORT && ++sub == parts) XT_BLOCK_DONE;
     }
-    if (++sub == subs) {   // the block is complete: max(round(c x)) = round(c max(x)) for c > 0, else mr is unused
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float v = swap32_max(a.c > 0.0f ? fmaxf(m[g], mr[g] * a.c) : m[g]);
-        const int64_t row = row0 + RG * (G * wave + g) + j / HPW;
-        if (h == 0 && bi < nblk[g])
-          store_score(a, (int64_t)head * a.s_hs + (q0 + row) * a.s_ns + (blk_lo + bi) * a.s_ks, v);
-        m[g] = mr[g] = -__builtin_inff();
-      }
-      sub = 0;
-      ++bi;
-    }
+    if (!SHORT && ++sub == parts) XT_BLOCK_DONE;
   }
+#undef XT_BLOCK_DONE
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -601,9 +612,9 @@ int score_common(const char* what, ScoreArgs& a, int dim, int q_dtype, const voi
 template <int NK, bool BF>
 int decode_dispatch(int T, const ScoreArgs& a, dim3 grid, hipStream_t st) {
   // The block-diagonal query fits the MFMA's rows. At 64 dims a block of 32 or 64 keys has fewer products than its
-  // reductions over the lanes, one per head, cost (heads x requests x keys, block size: this kernel / the other): 4 x 64
-  // x 32768, 32: 41.9 / 36.2 us; 4 x 16 x 4096, 64: 4.5 / 4.2; but 4 x 64 x 32768, 128: 36.2 / 44.4. At 128 dims it is
-  // ahead from 32 keys on (4 x 64 x 32768, 32: 49.8 / 50.1 us, 64: 48.4 / 49.3, 128: 52.8 / 60.0).
+  // reductions over the lanes, one per head, cost (heads x requests x keys, block size: this kernel / the other): 4 x
+  // 64 x 32768, 32: 41.9 / 36.2 us; 4 x 16 x 4096, 64: 4.5 / 4.2; but 4 x 64 x 32768, 128: 36.2 / 44.4. At 128 dims it
+  // is ahead from 32 keys on (4 x 64 x 32768, 32: 49.8 / 50.1 us, 64: 48.4 / 49.3, 128: 52.8 / 60.0).
   if (a.heads <= 32 / NK) {
     const dim3 block(64 * kScoreWaves);
     if constexpr (NK > 4) {
@@ -635,14 +646,23 @@ int decode_dispatch(int T, const ScoreArgs& a, dim3 grid, hipStream_t st) {
   return XT_OK;
 }
 
+template <int NK, int G, bool BF, bool SHORT>
+void prefill_launch(int hpw, const ScoreArgs& a, dim3 grid, hipStream_t st) {
+  const dim3 block(64 * kScoreWaves);
+  if (hpw == 1)
+    hipLaunchKernelGGL((prefill_scores_kernel<NK, 1, G, BF, SHORT>), grid, block, 0, st, a);
+  else if (hpw == 2)
+    hipLaunchKernelGGL((prefill_scores_kernel<NK, 2, G, BF, SHORT>), grid, block, 0, st, a);
+  else
+    hipLaunchKernelGGL((prefill_scores_kernel<NK, 4, G, BF, SHORT>), grid, block, 0, st, a);
+}
+
 template <int NK, int G, bool BF>
 void prefill_dispatch(int hpw, const ScoreArgs& a, dim3 grid, hipStream_t st) {
-  if (hpw == 1)
-    hipLaunchKernelGGL((prefill_scores_kernel<NK, 1, G, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
-  else if (hpw == 2)
-    hipLaunchKernelGGL((prefill_scores_kernel<NK, 2, G, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
+  if (a.block_size < kStageKeys<NK>)
+    prefill_launch<NK, G, BF, true>(hpw, a, grid, st);
   else
-    hipLaunchKernelGGL((prefill_scores_kernel<NK, 4, G, BF>), grid, dim3(64 * kScoreWaves), 0, st, a);
+    prefill_launch<NK, G, BF, false>(hpw, a, grid, st);
 }
 
 }  // namespace
