@@ -442,19 +442,22 @@ __global__ __launch_bounds__(64 * kScoreWaves, 2) void prefill_scores_kernel(con
   const int64_t whole = a.c > 0.0f ? max((int64_t)0, min(pre + row0 + 1, seq) - pos_lo) / (SHORT ? 32 : S) : 0;
   load_raw(slot_next);
   slot_next = slot_at(1);
-  float m[G], mr[G];   // scaled maxima of masked chunks, raw maxima of unmasked ones
+  // scaled maxima of masked chunks, raw maxima of unmasked ones (with c <= 0 there are none: c times none is -inf, or
+  // NaN)
+  float m[G], mr[G];
+  const float none = a.c > 0.0f ? -__builtin_inff() : __builtin_inff();
 #pragma unroll
-  for (int g = 0; g < G; ++g) m[g] = mr[g] = -__builtin_inff();
-  // The block is complete: max(round(c x)) = round(c max(x)) for c > 0, else mr is unused. (As a lambda it took registers
-  // from the long form's loop, 1 %.)
+  for (int g = 0; g < G; ++g) m[g] = -__builtin_inff(), mr[g] = none;
+  // The block is complete: max(round(c x)) = round(c max(x)) for c > 0. (As a lambda it took registers from the long
+  // form's loop, 1 %.)
 #define XT_BLOCK_DONE                                                                                                \
   do {                                                                                                               \
     _Pragma("unroll") for (int g = 0; g < G; ++g) {                                                                  \
-      const float v = swap32_max(a.c > 0.0f ? fmaxf(m[g], mr[g] * a.c) : m[g]);                                      \
+      const float v = swap32_max(fmaxf(m[g], mr[g] * a.c));                                                          \
       const int64_t row = row0 + RG * (G * wave + g) + j / HPW;                                                      \
       if (h == 0 && bi < nblk[g])                                                                                    \
         store_score(a, (int64_t)head * a.s_hs + (q0 + row) * a.s_ns + (blk_lo + bi) * a.s_ks, v);                    \
-      m[g] = mr[g] = -__builtin_inff();                                                                              \
+      m[g] = -__builtin_inff(), mr[g] = none;                                                                        \
     }                                                                                                                \
     sub = 0;                                                                                                         \
     ++bi;                                                                                                            \
