@@ -764,10 +764,13 @@ extern "C" int xt_minimax_prefill_scores(const void* q, int64_t q_token_stride, 
   const int64_t want_chunks = (max_blocks + 7) / 8;
   a.chunks = want_chunks < 1 ? 1 : want_chunks > 64 ? 64 : (int)want_chunks;
   a.chunk_blocks = max_blocks > 0 ? (int)((max_blocks + a.chunks - 1) / a.chunks) : 0x7FFFFFFF;
-  // four column groups per wavefront share each staged key where the query fits the registers and the row tiles
-  // still give every CU its two workgroups
+  // Four column groups per wavefront share each staged key where the query fits the registers and the row tiles still
+  // give every CU its two workgroups. At 64 dims a short block's products are fewer than what ends it, and two groups
+  // leave registers for twice the wavefronts (4 heads x 8192 rows against 38192 keys, blocks of 32, four / two: 352 /
+  // 299 us, 64: 247 / 225, against 8292 keys, 32: 63 / 47; 128: about even).
   const int64_t tiles4 = ((int64_t)max_q_len * hpw + 511) / 512;
-  const int G = dim <= 128 && tiles4 * a.chunks * batch >= 2 * device_cus() ? 4 : 2;
+  const bool wide = dim == 128 || (dim == 64 && block_size >= 128);
+  const int G = wide && tiles4 * a.chunks * batch >= 2 * device_cus() ? 4 : 2;
   const int rows = 128 * G / hpw;
   const int64_t tiles = (max_q_len + rows - 1) / rows;
   if (tiles * a.chunks > 0x7FFFFFFF) return fail(XT_EUNSUPPORTED, "%s: %lld query tiles", what, (long long)tiles);
