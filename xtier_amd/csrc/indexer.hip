@@ -676,11 +676,13 @@ __global__ __launch_bounds__(64 * kQsaWaves) void qsa_logits_kernel(const QsaArg
 // head sum beside it (from 8 heads on they are the larger part). 352 rows x 95088 keys, 4 heads x 128: 50.4 us (3.1
 // TB/s) against 91.8 us for the kernel above, whose wavefronts each read the keys from L2 and wait for their stores
 // with them; 352 x 65536: 8 heads 128 -> 61 us, 16 heads 261 -> 99, 32 heads 590 -> 188.
-// The stores are non-temporal: the logits alone take 50.4 us in place of 60.5 at 352 x 95088. With the selection of
-// 2048 positions behind them (4 heads, plain -> non-temporal): 352 x 4100 keys 23.0 -> 21.6 us, 352 x 32768 48.3 ->
-// 47.5, 32 x 65536 29.7 -> 29.3; but 32 x 4100 13.9 -> 14.4, and from about 60 MB of logits on the selection, which
-// then reads them from HBM, loses more than the stores gain (352 x 65536 78.3 -> 79.4, x 95088 104.5 -> 109.5; 512 x
-// 95088 129 -> 137).
+// With four column groups (32 MB of logits and more at 4 heads) the stores are non-temporal: the logits alone take
+// 50.4 us in place of 60.5 at 352 x 95088. With the selection of 2048 positions behind them 352 x 32768 takes 48.3 ->
+// 47.5 us, but from about 60 MB on the selection, which then reads them from HBM, loses more than the stores gain (352
+// x 65536 78.3 -> 79.4, x 95088 104.5 -> 109.5; 512 x 95088 129 -> 137). With fewer groups they are of device scope,
+// which passes them on without waiting for the end of the kernel and leaves them to the selection (4 heads, plain /
+// non-temporal / device scope, alone 32 x 4100 4.7 / 5.1 / 4.6 us, 352 x 4100 10.2 / 10.0 / 9.3; with the selection 32
+// x 4100 13.9 / 14.4 / 13.8, 352 x 4100 23.0 / 21.6 / 21.0, 32 x 65536 29.7 / 29.3 / 28.9).
 template <int NK, int G>
 constexpr int kQsaStage = (NK <= 8 ? 64 : 32) * (G == 4 ? 2 : 1);   // keys per stage
 
@@ -691,6 +693,7 @@ __global__ __launch_bounds__(64 * kQsaWaves, 2) void qsa_logits_lds_kernel(const
   constexpr int kRowsG = 32 / H, kRowsW = G * kRowsG, kRowsWg = kQsaWaves * kRowsW;
   constexpr int kPieces = S * 2 * NK / (64 * kQsaWaves);   // 16-byte pieces a thread stages
   constexpr int kOut = H <= 4 ? 16 / H : H == 32 ? 1 : 16 / H;   // logits per lane and column group
+  constexpr int kStorePolicy = G == 4 ? 2 : 16;    // non-temporal; device scope
   __shared__ __align__(16) uint16_t lds[2][S * ROW];
   __shared__ int2 range[kRowsWg];   // [start, end) of the rows (read behind the loop's first barrier)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
@@ -831,7 +834,7 @@ __global__ __launch_bounds__(64 * kQsaWaves, 2) void qsa_logits_lds_kernel(const
 #pragma unroll
         for (int o = 0; o < kOut; ++o)
           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[o]), rsrc,
-                                              (int)(koff + (uint32_t)(g * kRowsG + first(o)) * row_step), 0, 2);
+                                              (int)(koff + (uint32_t)(g * kRowsG + first(o)) * row_step), 0, kStorePolicy);
       }
     }
   }
