@@ -139,6 +139,18 @@ def test_row_arguments_of_rows_past_the_last_end(batch, extra, given):
         assert (x[len(r):] == y).all()
 
 
+@pytest.mark.parametrize('given', [True, False])
+def test_queries_past_the_last_end_are_zero(given):
+    """Rows of no request attend to nothing; the others are as without them."""
+    c = _case(83, q_lens=(70, 41), prefix=(300, 129), bq=16, topk=3)
+    pool = _pages(8, 48)
+    if not given:
+        c['cu_blk'] = None
+    plain = _run(c, pool)
+    padded = _run(dict(c, q=torch.cat([c['q'], c['q'][:37]])), pool)
+    assert torch.equal(padded[:111], plain) and not padded[111:].any()
+
+
 def test_strided_pool_kv_scale_and_queries_without_keys():
     print('block-sparse prefill: strided pool, kv_scale, empty rows', flush=True)
     c = _case(77, q_lens=(40, 70), prefix=(300, 129), bq=16, topk=3)

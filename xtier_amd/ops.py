@@ -541,10 +541,10 @@ def fp4_prefill_gqa_share_sparse(q, k_cache, v_cache, sink, req_to_token, slot_i
     BF16, request b's queries are rows cu_seqlens[b] .. cu_seqlens[b+1]-1 at positions prefix_lens[b] + i; the
     queries of one block of block_size_q share the block list topk_idx[kh, cu_seqblocks_q[b] + i // block_size_q, :]
     (block ids of block_size_k tokens, -1 padded); k_cache / v_cache payload pages, k_sc / v_sc their scale bytes.
-    Returns o [total_q, qh, d] in q's dtype. Lengths are clamped to req_to_token.shape[1]; a key block wholly after a
-    query's position adds nothing to its softmax (the reference's running max starts at -inf, so such a block listed
-    first gives it NaN). use_tma / num_warps / num_stages / max_seqblock_q are accepted for the reference's signature
-    and ignored."""
+    Returns o [total_q, qh, d] in q's dtype (zeros for rows of no request). Lengths are clamped to
+    req_to_token.shape[1]; a key block wholly after a query's position adds nothing to its softmax (the reference's
+    running max starts at -inf, so such a block listed first gives it NaN). use_tma / num_warps / num_stages /
+    max_seqblock_q are accepted for the reference's signature and ignored."""
     assert sink is None and loc_mapping is None and block_size_k == k_cache.shape[2]
     k_pay, k_sc8 = _pages(k_cache, k_sc, 'fp4_prefill_gqa_share_sparse')
     v_pay, v_sc8 = _pages(v_cache, v_sc, 'fp4_prefill_gqa_share_sparse')
